@@ -215,7 +215,8 @@ __global__ void __launch_bounds__(kPfWG) pf_router(const float *x, uint32_t T, c
 // token's window mask for the dispatch.
 
 __global__ void __launch_bounds__(kPfWG) pf_topk(const float *logits, uint32_t T, uint32_t E, uint32_t K,
-                                                 int32_t *ids, float *w, float *gs, unsigned long long *masks) {
+                                                 int32_t *ids, float *w, float *gs, unsigned long long *masks,
+                                                 int32_t *ids_out, float *w_out) {
   __shared__ uint64_t tab[32];
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
   __syncthreads();
@@ -232,6 +233,8 @@ __global__ void __launch_bounds__(kPfWG) pf_topk(const float *logits, uint32_t T
     ids[(uint64_t)t * K + lane] = (int32_t)my_id;
     w[(uint64_t)t * K + lane] = wk;
     atomicOr(&masks[(uint64_t)(t / 64) * E + my_id], 1ull << (t % 64));  // the dispatch's window mask
+    if (ids_out) ids_out[(uint64_t)t * K + lane] = (int32_t)my_id;        // the caller's copies
+    if (w_out) w_out[(uint64_t)t * K + lane] = wk;
   }
   if (lane == 0 && gs) gs[t] = sigmoid_libm(lg[E], tab);
 }
@@ -457,7 +460,8 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
                                                       const uint16_t *xb, const float *xn, const int *xlsb, uint32_t T,
                                                       uint32_t E, uint32_t H, uint32_t K, const float *bias,
                                                       float gamma_rmax, float bias_max, int32_t *ids, float *w,
-                                                      unsigned long long *masks, uint32_t *cnt_exact) {
+                                                      unsigned long long *masks, uint32_t *cnt_exact,
+                                                      int32_t *ids_out, float *w_out) {
   __shared__ uint64_t tab[32];
   __shared__ uint32_t cand[kPfWG / 64][kMaxRouteExperts];
   __shared__ uint32_t xkey[kPfWG / 64][kMaxRouteExperts];  // 0, or an exactly summed expert's key (cleared after)
@@ -587,6 +591,8 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
     ids[(uint64_t)t * K + lane] = (int32_t)my_id;
     w[(uint64_t)t * K + lane] = wk;
     atomicOr(&masks[(uint64_t)(t / 64) * E + my_id], 1ull << (t % 64));
+    if (ids_out) ids_out[(uint64_t)t * K + lane] = (int32_t)my_id;  // the caller's copies
+    if (w_out) w_out[(uint64_t)t * K + lane] = wk;
   }
 }
 
@@ -1605,8 +1611,8 @@ hipError_t routed_experts(const PfShape &S, const PfLayer &L, const PfBufs &b, h
 
 }  // namespace
 
-hipError_t prefill_forward(const PfShape &S, const PfLayer &L, const PfBufs &b, const float *x, float *y, hipStream_t st,
-                     const PfHook &hook) {
+hipError_t prefill_forward(const PfShape &S, const PfLayer &L, const PfBufs &b, const float *x, float *y, int32_t *ids_out,
+                           float *w_out, hipStream_t st, const PfHook &hook) {
   const uint32_t H = S.H, F = S.F, E = S.E, K = S.K, T = S.T, Ug = units_of(H), Ud = units_of(F);
   const uint32_t xr = quant_vec_dot_type(S.gate_type);
   const uint32_t xs = S.has_shared ? quant_vec_dot_type(S.sh_gate_type) : xr;
@@ -1673,7 +1679,8 @@ hipError_t prefill_forward(const PfShape &S, const PfLayer &L, const PfBufs &b, 
     }
     {
       HookScope k(hook, "pf_topk", st);
-      pf_topk<<<(T + 3) / 4, kPfWG, 0, st>>>(b.logits, T, E, K, b.ids, b.w, S.has_shared ? b.gs : nullptr, b.masks);
+      pf_topk<<<(T + 3) / 4, kPfWG, 0, st>>>(b.logits, T, E, K, b.ids, b.w, S.has_shared ? b.gs : nullptr, b.masks,
+                                           ids_out, w_out);
     }
   } else {
     {
@@ -1693,7 +1700,7 @@ hipError_t prefill_forward(const PfShape &S, const PfLayer &L, const PfBufs &b, 
       const float gamma = (float)(1.01 * (31 + H / 128 + 3) * 0x1p-23);
       pf_topk_cert<<<(T + 3) / 4, kPfWG, 0, st>>>(b.logits, L.router, L.rlsb, b.xb, b.xn, b.xlsb, T, E, H, K, L.bias,
                                                   gamma * L.rmax * 1.0001f, L.bias_max, b.ids, b.w,
-                                                  b.masks, b.cnt_exact);
+                                                  b.masks, b.cnt_exact, ids_out, w_out);
     }
   }
   if (S.has_shared && hipStreamWaitEvent(st, b.xq, 0) != hipSuccess) return hipGetLastError();

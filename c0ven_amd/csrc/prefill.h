@@ -88,9 +88,9 @@ constexpr uint32_t pf_max_tiles(uint32_t T, uint32_t K, uint32_t E) { return (T 
 constexpr uint32_t pf_windows(uint32_t T) { return (T + 63) / 64; }
 
 // Enqueues the block for s.T tokens of x (T x H fp32, rows contiguous, device) into y (the same shape); returns the
-// launches' error state.
-hipError_t prefill_forward(const PfShape &s, const PfLayer &L, const PfBufs &b, const float *x, float *y, hipStream_t st,
-                     const PfHook &hook);
+// launches' error state. ids_out and w_out (T x K, either may be null) receive the routing beside b.ids and b.w.
+hipError_t prefill_forward(const PfShape &s, const PfLayer &L, const PfBufs &b, const float *x, float *y,
+                           int32_t *ids_out, float *w_out, hipStream_t st, const PfHook &hook);
 // Pre-routed (CpuExperts::compute_many's jobs): b.ids and b.w already hold s.T x s.K ranks (ids < 0 where a token has
 // fewer jobs; s.K at most the scratch's width); no router, no shared expert. y[t] = the token's jobs in rank order.
 hipError_t prefill_jobs(const PfShape &s, const PfLayer &L, const PfBufs &b, const float *x, float *y, hipStream_t st,
