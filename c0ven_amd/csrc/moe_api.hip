@@ -223,6 +223,8 @@ struct moe_ctx {
   HcBufs hcp{};                 // the prefill mix's scratch (hc_lr > 0 and max_tokens > the decode kernel's)
   uint8_t *codebooks = nullptr;  // the caller's iq2s_grid and iq3xxs_grid (QGRID layout, up to QGRID_IQ3S)
   bool have_codebooks = false;
+  uint8_t *coded = nullptr;      // the same as levels (PfLayer::coded), when coded_ok
+  bool coded_ok = false;
   const void *kernel = nullptr;  // moe_decode for the context's set of weight types
   const void *kernel_hc = nullptr;  // the same with the hyper-connection items (hc_lr > 0)
   uint32_t grid_hc = 0;
@@ -308,6 +310,22 @@ void validate(const moe_config &c) {
   require(c.max_tokens <= kMaxPrefillTokens, "max_tokens must be at most 16384");
   require(c.swiglu_limit >= 0.0f, "swiglu_limit must be >= 0");
   require(c.hc_lr <= kHcMaxLr && c.hc_lr % 8 == 0, "hc_lr must be a multiple of 8, at most 512");
+}
+
+// A codebook table's bytes as indices of its distinct byte values (levels, in order of first use): ggml's iq2s_grid has
+// three and iq3xxs_grid eight. False when there are more than `most`, or one is outside 0..127.
+bool code_levels(const uint8_t *table, uint32_t n, uint32_t most, uint8_t *out, uint8_t *levels) {
+  uint32_t count = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    uint32_t l = 0;
+    while (l < count && levels[l] != table[i]) l++;
+    if (l == count) {
+      if (count == most || table[i] > 127) return false;
+      levels[count++] = table[i];
+    }
+    out[i] = (uint8_t)l;
+  }
+  return true;
 }
 
 // Types that decode through the caller's codebooks need them set first.
@@ -448,7 +466,8 @@ void forward_dev(moe_ctx *c, uint32_t layer, const float *x, uint32_t T, float *
     PfShape S{g.n_embd, g.n_ff, g.n_expert, K, T, g.gate_type, g.down_type, g.sh_gate_type, g.sh_down_type,
               g.has_shared, g.swiglu_limit, g.sh_up_type, (g.flags & MOE_FLAG_EXACT_ROUTER) ? 1u : 0u};
     PfLayer PL{L.router, L.router_t, L.has_bias ? L.bias : nullptr, L.experts, c->ex_bytes, c->ex_up, c->ex_down, L.shared,
-               c->sh_up, c->sh_down, c->codebooks, L.rlsb, L.rmax, L.bias_max};
+               c->sh_up, c->sh_down, c->codebooks,
+               c->coded_ok ? c->coded : nullptr, L.rlsb, L.rmax, L.bias_max};
     PfHook hook{c->timing ? timing_hook : nullptr, c};
     check(prefill_forward(S, PL, c->pf, x, y, direct ? ids : nullptr, direct ? w : nullptr, s, hook), "prefill launch");
     c->last_ids = c->pf.ids, c->last_w = c->pf.w, c->last_pf_T = T;
@@ -590,6 +609,8 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
       // Up to kMaxExperts experts: a layer's, or a pre-routed call's borrowed ones.
       b.tiles = c->alloc<MoeTile>(pf_max_tiles(TM, K, kMaxExperts));
       b.ntiles = c->alloc<uint32_t>(1);
+      for (auto &sp : b.spans) sp = c->alloc<MoeTile>(pf_max_spans(TM, K, kMaxExperts, kPfSpanMin));
+      b.nspans = c->alloc<uint32_t>(2);
       b.masks = c->alloc<unsigned long long>((uint64_t)pf_windows(TM) * kMaxExperts);
       b.h = c->alloc<float>(A2 * F);
       b.hact = c->alloc<uint8_t>(A2 * Ud * kActBytes);
@@ -630,6 +651,7 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
     c->flags = c->alloc<uint64_t>(kFlagCount);
     check(hipMemset(c->flags, 0, kFlagCount * sizeof(uint64_t)), "hipMemset");
     c->codebooks = c->alloc<uint8_t>(QGRID_IQ3S);
+    c->coded = c->alloc<uint8_t>(QGRID_IQ3S + 16);
     if (g.hc_lr) {
       c->hc_n = c->alloc<float>((uint64_t)T * kHcStreams * H);
       c->hc_l = c->alloc<float>((uint64_t)T * (g.hc_lr + kHcStreams));
@@ -1130,7 +1152,8 @@ MOE_API moe_status moe_compute_many(moe_ctx *c, const moe_cm_job *jobs, uint32_t
       check(hipMemcpyAsync(c->pf.w, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice, s), "w");
       PfShape S{H, F, c->bc_slots, K, ntok, g.gate_type, g.down_type, g.sh_gate_type, g.sh_down_type, 0, g.swiglu_limit,
                 g.sh_up_type};
-      PfLayer PL{nullptr, nullptr, nullptr, c->bc_base, c->ex_bytes, c->ex_up, c->ex_down, nullptr, 0, 0, c->codebooks, nullptr, 0.0f, 0.0f};
+      PfLayer PL{nullptr, nullptr, nullptr, c->bc_base, c->ex_bytes, c->ex_up, c->ex_down, nullptr, 0, 0, c->codebooks,
+                 c->coded_ok ? c->coded : nullptr, nullptr, 0.0f, 0.0f};
       PfHook hook{c->timing ? timing_hook : nullptr, c};
       check(prefill_jobs(S, PL, c->pf, c->x_dev, c->y_dev, s, hook), "prefill launch");
       c->last_ids = c->pf.ids, c->last_w = c->pf.w, c->last_pf_T = ntok;
@@ -1398,6 +1421,11 @@ MOE_API moe_status moe_set_codebooks(moe_ctx *c, const uint8_t *qgrid, uint64_t 
     require(std::memcmp(qgrid + QGRID_IQ3S, kIq3sGridHost, sizeof kIq3sGridHost) == 0,
             "the buffer's IQ3_S region is not ggml's iq3s_grid: not a QGRID-layout codebook buffer");
     check(hipMemcpy(c->codebooks, qgrid, QGRID_IQ3S, hipMemcpyHostToDevice), "upload codebooks");
+    std::vector<uint8_t> coded(QGRID_IQ3S + 16, 0);
+    c->coded_ok = code_levels(qgrid + QGRID_IQ2S, QGRID_IQ3XXS - QGRID_IQ2S, 4, coded.data() + QGRID_IQ2S, coded.data() + QGRID_IQ3S) &&
+                  code_levels(qgrid + QGRID_IQ3XXS, QGRID_IQ3S - QGRID_IQ3XXS, 8, coded.data() + QGRID_IQ3XXS,
+                              coded.data() + QGRID_IQ3S + 8);
+    if (c->coded_ok) check(hipMemcpy(c->coded, coded.data(), coded.size(), hipMemcpyHostToDevice), "upload coded codebooks");
     c->have_codebooks = true;
   });
 }

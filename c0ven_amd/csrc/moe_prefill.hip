@@ -7,6 +7,7 @@
 // do, and add a row's units in sequence, as the oracle does.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "act_quant.h"
@@ -639,6 +640,15 @@ __device__ __forceinline__ uint32_t block_scan512(uint32_t v, uint32_t *wsum) {
   return v + add;
 }
 
+// The span lists pf_place writes beside the tiles: positions a span (0: none; at most 16 kSpanClasses), the records,
+// their counts. The longest spans come first, so that the last work-groups of a launch are short ones.
+constexpr uint32_t kSpanClasses = 16;
+struct PfSpans {
+  uint32_t len[2];
+  MoeTile *list[2];
+  uint32_t *n;
+};
+
 constexpr uint32_t kScanBatch = 32;  // window masks a thread holds at once (all of them up to 2048 tokens)
 
 // One work-group a window. Thread e counts expert e's assignments in every window (the masks' popcounts, all loaded
@@ -648,8 +658,8 @@ constexpr uint32_t kScanBatch = 32;  // window masks a thread holds at once (all
 // rows) and their count.
 __global__ void __launch_bounds__(kDispWG) pf_place(const int32_t *ids, uint32_t T, uint32_t K, uint32_t E,
                                                     uint32_t nwin, const unsigned long long *masks, MoeTile *tiles,
-                                                    uint32_t *ntiles, uint32_t *perm, uint32_t *inv) {
-  __shared__ uint32_t wsum[kDispWG / 64], start[kDispWG];
+                                                    uint32_t *ntiles, uint32_t *perm, uint32_t *inv, PfSpans sp) {
+  __shared__ uint32_t wsum[kDispWG / 64], start[kDispWG], hist[kSpanClasses + 2];
   __shared__ unsigned long long mine[kDispWG];
   const uint32_t w = blockIdx.x, e = threadIdx.x, ec = min(e, E - 1);
   uint32_t c = 0, before = 0;
@@ -677,6 +687,32 @@ __global__ void __launch_bounds__(kDispWG) pf_place(const int32_t *ids, uint32_t
         tiles[t0 + i] = m;
       }
     if (e == E - 1) *ntiles = t0 + nt;
+#pragma unroll
+    for (uint32_t v = 0; v < 2; v++) {  // the same positions in the GEMMs' spans, the longest first
+      const uint32_t P = sp.len[v];
+      if (P == 0) continue;
+      const uint32_t full = c / P, rem = c % P, k = (rem + 15) / 16;  // whole spans, then the rest by position tiles
+      const uint32_t f0 = block_scan512(full, wsum) - full;
+      if (e < kSpanClasses + 1) hist[e] = 0u;
+      if (e == kDispWG - 1) hist[kSpanClasses + 1] = f0 + full;  // all whole spans
+      __syncthreads();
+      const uint32_t at = rem ? atomicAdd(&hist[k], 1u) : 0u;
+      __syncthreads();
+      uint32_t before_k = hist[kSpanClasses + 1], all = before_k;
+      for (uint32_t i = 1; i <= kSpanClasses; i++) all += hist[i], before_k += i > k ? hist[i] : 0u;
+      if (e < E) {
+        MoeTile m;
+        m.expert = e, m.slot = e, m.count = P;
+        for (uint32_t i = 0; i < full; i++) {
+          m.start = base + P * i;
+          sp.list[v][f0 + i] = m;
+        }
+        m.start = base + P * full, m.count = rem;
+        if (rem) sp.list[v][before_k + at] = m;
+      }
+      if (e == 0) sp.n[v] = all;
+      __syncthreads();
+    }
   }
   __syncthreads();
   const uint32_t t0 = 64 * w, a0 = t0 * K, a1 = min(T, t0 + 64) * K;
@@ -698,7 +734,7 @@ struct PfGemm {
   const uint32_t *ntiles;
   uint32_t shared_T;       // > 0: the shared expert over tokens 0 .. shared_T - 1 in order (implicit tiles)
   const uint32_t *perm;    // routed gate/up: position -> assignment (token = assignment / K)
-  uint32_t K;
+  uint32_t K;              // (pf_down_q8: values of a row)
   const uint8_t *act;      // activation units: by token (gate/up) or by position (down)
   uint32_t act_by_pos;
   const uint8_t *mat;      // expert e's matrix at mat + e * stride; up at + up_off
@@ -710,6 +746,9 @@ struct PfGemm {
   uint32_t rb_span;        // pf_gemm16 Q4_K down: consecutive 64-row blocks a work-group (> 1 only when U <= 2)
   uint32_t U;              // 256-value units of K (a partial last one padded with zeros)
   const uint8_t *codebooks;  // the caller's codebooks (QGRID layout) for IQ3_XXS and IQ2_S
+  const uint8_t *coded;      // the same as levels (PfLayer::coded)
+  const MoeTile *spans;    // pf_gate_up_planes, pf_down_q8: the experts' positions in runs of at most plane_pos, kDownPos
+  const uint32_t *nspans;
 };
 
 // Rows of one grid.y step of the (tiles x row groups) grid the host computes: 64 of gate and of up, or 128 of down.
@@ -1411,6 +1450,25 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
     }
 }
 
+// Work-group b of a span launch: span *sp's row group *rb (nrb a span). XCD x (b % 8) takes spans x, x + 8, ..., a span's
+// row groups one after another, so a span's activations are read into one XCD's L2 and, the list being longest first, the
+// XCDs get equal work. The grid is span_grid(most spans, nrb); false past the last span.
+__device__ __forceinline__ bool span_item(uint32_t b, uint32_t nrb, uint32_t nspans, uint32_t *sp, uint32_t *rb) {
+  const uint32_t j = b / 8;
+  *sp = (j / nrb) * 8 + b % 8, *rb = j % nrb;
+  return *sp < nspans;
+}
+constexpr uint32_t span_grid(uint32_t spans, uint32_t nrb) { return (spans + 7) / 8 * 8 * nrb; }
+
+}  // namespace
+}  // namespace c0ven
+
+#include "pf_planes.h"
+#include "pf_down.h"
+
+namespace c0ven {
+namespace {
+
 // Positions a gate/up work-group takes for a weight type (the kernel's kPos).
 constexpr uint32_t gu_pos(uint32_t) { return MOE_TILE; }
 // The gate/up types that run on pf_gate_up_q4k / pf_gate_up_iq3s (gate and up of a row in one wave); the others on
@@ -1527,6 +1585,47 @@ void launch_gemm(uint32_t type, uint32_t U, dim3 grid, const PfGemm &g, hipStrea
     pf_gemm16<QT_Q8_0, kGU><<<g2, kPfWG, 0, s>>>(q);
 }
 
+// Routed gate/up on pf_gate_up_planes, spans of plane_len positions (0: the type's codebook has no levels, or Q5_K, Q6_K and
+// the q8_0 family): at most ns of them, F rows of each matrix.
+uint32_t plane_len(uint32_t type, const uint8_t *coded) {
+  switch (type) {
+    case QT_Q4_K: return plane_pos<QT_Q4_K>();
+    case QT_IQ3_S: return plane_pos<QT_IQ3_S>();
+    case QT_IQ4_XS: return plane_pos<QT_IQ4_XS>();
+    case QT_IQ3_XXS: return coded ? plane_pos<QT_IQ3_XXS>() : 0u;
+    case QT_IQ2_S: return coded ? plane_pos<QT_IQ2_S>() : 0u;
+    default: return 0u;
+  }
+}
+void launch_planes(uint32_t type, uint32_t U, uint32_t ns, uint32_t F, const PfGemm &g, hipStream_t s) {
+  PfGemm q = g;
+  q.U = U;
+  q.row_blocks = F / 64;
+  const dim3 grid(span_grid(ns, q.row_blocks));
+  switch (type) {
+    case QT_Q4_K: pf_gate_up_planes<QT_Q4_K><<<grid, kPfWG, 0, s>>>(q); break;
+    case QT_IQ3_S: pf_gate_up_planes<QT_IQ3_S><<<grid, kPfWG, 0, s>>>(q); break;
+    case QT_IQ3_XXS: pf_gate_up_planes<QT_IQ3_XXS><<<grid, kPfWG, 0, s>>>(q); break;
+    case QT_IQ2_S: pf_gate_up_planes<QT_IQ2_S><<<grid, kPfWG, 0, s>>>(q); break;
+    default: pf_gate_up_planes<QT_IQ4_XS><<<grid, kPfWG, 0, s>>>(q); break;
+  }
+}
+
+// Routed down of the q8_0 family on pf_down_q8 (spans of kDownPos positions), H rows of F values.
+constexpr bool down_q8(uint32_t type, uint32_t F) { return q8_family(type) && down_lds(F) <= kDownMaxLds; }
+void launch_down_q8(uint32_t type, uint32_t F, uint32_t ns, uint32_t H, const PfGemm &g, hipStream_t s) {
+  PfGemm q = g;
+  q.U = units_of(F), q.K = F, q.row_blocks = H / 64;
+  // The kernel picks its row groups a work-group (down_walk) from the spans there are: at most this many work-groups.
+  const dim3 grid(std::max(2 * kDownGroups, span_grid(ns, q.row_blocks / 8)));
+  if (type == QT_IQ4_NL)
+    pf_down_q8<QT_IQ4_NL><<<grid, kPfWG, down_lds(F), s>>>(q);
+  else if (type == QT_Q2_0)
+    pf_down_q8<QT_Q2_0><<<grid, kPfWG, down_lds(F), s>>>(q);
+  else
+    pf_down_q8<QT_Q8_0><<<grid, kPfWG, down_lds(F), s>>>(q);
+}
+
 struct HookScope {
   const PfHook &h;
   const char *name;
@@ -1561,6 +1660,14 @@ C0VEN_PF_GEMM16(QT_IQ4_XS)
 C0VEN_PF_GEMM16(QT_Q5_K)
 C0VEN_PF_GEMM16(QT_Q6_K)
 #undef C0VEN_PF_GEMM16
+template __global__ void pf_gate_up_planes<QT_Q4_K>(PfGemm);
+template __global__ void pf_gate_up_planes<QT_IQ3_S>(PfGemm);
+template __global__ void pf_gate_up_planes<QT_IQ3_XXS>(PfGemm);
+template __global__ void pf_gate_up_planes<QT_IQ2_S>(PfGemm);
+template __global__ void pf_gate_up_planes<QT_IQ4_XS>(PfGemm);
+template __global__ void pf_down_q8<QT_IQ4_NL>(PfGemm);
+template __global__ void pf_down_q8<QT_Q2_0>(PfGemm);
+template __global__ void pf_down_q8<QT_Q8_0>(PfGemm);
 template void launch_gemm<false>(uint32_t, uint32_t, dim3, const PfGemm &, hipStream_t);
 template void launch_gemm<true>(uint32_t, uint32_t, dim3, const PfGemm &, hipStream_t);
 
@@ -1578,11 +1685,15 @@ hipError_t routed_experts(const PfShape &S, const PfLayer &L, const PfBufs &b, h
   const uint32_t hr = quant_vec_dot_type(S.down_type);
   const uint32_t halfwaves = kPfWG / 32;
   const uint32_t mt = pf_max_tiles(T, K, E);
+  // Span lists of the gate/up's and the down's lengths (one list where they agree).
+  const uint32_t lg = plane_len(S.gate_type, L.coded), ld = down_q8(S.down_type, F) ? kDownPos : 0u;
+  const PfSpans sp{{lg, ld == lg ? 0u : ld}, {b.spans[0], b.spans[1]}, b.nspans};
+  const uint32_t dl = ld == lg ? 0u : 1u;  // the down's list
   {
     HookScope k(hook, "pf_dispatch", st);
     const uint32_t nwin = pf_windows(T);
     if (!masks_built) pf_masks<<<nwin, kDispWG, 0, st>>>(b.ids, T, K, E, b.masks);
-    pf_place<<<nwin, kDispWG, 0, st>>>(b.ids, T, K, E, nwin, b.masks, b.tiles, b.ntiles, b.perm, b.inv);
+    pf_place<<<nwin, kDispWG, 0, st>>>(b.ids, T, K, E, nwin, b.masks, b.tiles, b.ntiles, b.perm, b.inv, sp);
   }
   {
     HookScope k(hook, "pf_gate_up", st);
@@ -1591,7 +1702,11 @@ hipError_t routed_experts(const PfShape &S, const PfLayer &L, const PfBufs &b, h
     g.mat = L.experts, g.stride = L.ex_bytes, g.up_off = L.ex_up_off, g.out = b.h, g.out_ld = F;
     g.codebooks = L.codebooks;
     g.limit = S.swiglu_limit;
-    launch_gate_up(S.gate_type, g, T, F, Ug, mt, st);
+    g.coded = L.coded, g.spans = b.spans[0], g.nspans = b.nspans;
+    if (lg)
+      launch_planes(S.gate_type, Ug, pf_max_spans(T, K, E, lg), F, g, st);
+    else
+      launch_gate_up(S.gate_type, g, T, F, Ug, mt, st);
   }
   {
     HookScope k(hook, "pf_quant_h", st);
@@ -1604,7 +1719,11 @@ hipError_t routed_experts(const PfShape &S, const PfLayer &L, const PfBufs &b, h
     g.tiles = b.tiles, g.ntiles = b.ntiles, g.K = K, g.act = b.hact, g.act_by_pos = 1;
     g.mat = L.experts + L.ex_down_off, g.stride = L.ex_bytes, g.out = b.y_asg, g.out_ld = H;
     g.codebooks = L.codebooks;
-    launch_gemm<false>(S.down_type, Ud, dim3(mt, H / gemm_rows<false>()), g, st);
+    g.spans = b.spans[dl], g.nspans = b.nspans + dl;
+    if (ld)
+      launch_down_q8(S.down_type, F, pf_max_spans(T, K, E, ld), H, g, st);
+    else
+      launch_gemm<false>(S.down_type, Ud, dim3(mt, H / gemm_rows<false>()), g, st);
   }
   return hipGetLastError();
 }

@@ -11,12 +11,13 @@
 //   pf_place       counting sort of the T k assignments by expert (stable: token order within an expert) into
 //                  MoeTile[] of at most MOE_TILE rows, perm (position -> assignment) and inv (assignment -> position)
 //                  (pre-routed ids: pf_masks builds the masks first)
-//   gate/up        per tile: gate and up on int8 MFMA, exact int32 block sums, the blocks' integer scales and the
-//                  unit's fp32 term in the oracle's order, SwiGLU. Q4_K: pf_gate_up_q4k, IQ3_S: pf_gate_up_iq3s (64
-//                  rows of each a work-group); the other types: pf_gemm16 (32 rows of each); activations loaded
-//                  straight to LDS
+//   gate/up        gate and up on int8 MFMA, exact integer unit sums and the unit's fp32 term in the oracle's order, SwiGLU.
+//                  Routed Q4_K, IQ3_S, IQ3_XXS, IQ2_S and IQ4_XS: pf_gate_up_planes (pf_planes.h: two int8 planes, spans of 64
+//                  or 128 of an expert's positions); the shared expert's Q4_K and IQ3_S: pf_gate_up_q4k, pf_gate_up_iq3s;
+//                  the rest: pf_gemm16 (per MoeTile); activations loaded straight to LDS
 //   pf_quant_rows  h -> the down's activation units
-//   down           per tile: the same kernels (64 or 128 rows a work-group)
+//   down           routed Q8_0, IQ4_NL and Q2_0: pf_down_q8 (pf_down.h: spans of 64 positions held in LDS); the rest:
+//                  pf_gemm16 (per MoeTile, 64 or 128 rows a work-group)
 //   pf_combine     y_t = sum_k w_k y_(t,k) in rank order + gs_t s_t
 // The shared expert runs through the same GEMMs over the tokens in order.
 #pragma once
@@ -46,6 +47,9 @@ struct PfLayer {
   const uint8_t *shared;
   uint64_t sh_up_off, sh_down_off;
   const uint8_t *codebooks;  // the caller's codebooks (QGRID layout) for IQ3_XXS and IQ2_S
+  const uint8_t *coded;      // the same tables with each byte as its level among the table's byte values, in place of them
+                             // (iq2s_grid at QGRID_IQ2S, iq3xxs_grid at QGRID_IQ3XXS), then at QGRID_IQ3S iq2s_grid's
+                             // four levels and at + 8 iq3xxs_grid's eight; null where a table has more, or one past 127
   const int *rlsb;           // per routed row: the least lsb of its bf16 values (the exact-sum condition)
   float rmax;                // the largest ||W_e||_2 over the routed rows (bf16 values), rounded up
   float bias_max;            // the largest |bias_e| (0 without a bias)
@@ -65,6 +69,8 @@ struct PfBufs {
   uint32_t *perm, *inv;    // Tmax K
   MoeTile *tiles;          // Tmax K / MOE_TILE + E
   uint32_t *ntiles;        // 1
+  MoeTile *spans[2];       // the same positions in spans of at least kPfSpanMin (pf_max_spans records each)
+  uint32_t *nspans;        // 2
   unsigned long long *masks;  // windows x E: the tokens of each 64-token window that chose each expert
   float *h, *h_sh;         // Tmax K x F (expert order), Tmax x F
   float *h_sh_up;          // Tmax x F: the shared up's rows when its type differs from the gate's (h_sh holds gate's)
@@ -84,6 +90,9 @@ struct PfHook {
 };
 
 constexpr uint32_t pf_max_tiles(uint32_t T, uint32_t K, uint32_t E) { return (T * K + MOE_TILE - 1) / MOE_TILE + E; }
+// Spans of P positions that T K assignments to E experts can make; the least P a GEMM's spans take.
+constexpr uint32_t kPfSpanMin = 64;
+constexpr uint32_t pf_max_spans(uint32_t T, uint32_t K, uint32_t E, uint32_t P) { return (T * K + P - 1) / P + E; }
 // 64-token windows of the dispatch's masks.
 constexpr uint32_t pf_windows(uint32_t T) { return (T + 63) / 64; }
 

@@ -39,10 +39,16 @@ __device__ __forceinline__ const T *field(const uint8_t *tile, uint32_t base, ui
   return (const T *)(tile + (uint64_t)base * nl) + (uint64_t)p * nl + idx;
 }
 
+// Byte j of a four-bit nibble's spread: bit j.
+__device__ __forceinline__ uint32_t sign_bits(uint32_t nib) { return (nib * 0x00204081u) & 0x01010101u; }
+// 0xff in the bytes of x that are 1, 0 in those that are 0: a byte permute whose selectors are the constants 0x0c (0x00)
+// and 0x0d (0xff). (x << 8) - x, which the compiler turns into a 32-bit multiply by 255, takes a quarter-rate
+// instruction: 16 of them a unit and matrix were 64 of the 385 VALU slots of an IQ2_S decode.
+__device__ __forceinline__ uint32_t sign_mask(uint32_t x) { return __builtin_amdgcn_perm(0u, 0u, x | 0x0c0c0c0cu); }
 // Bytes of g (each at least 1) negated where the matching bit of the four-bit nibble is set, without carries.
 __device__ __forceinline__ uint32_t sign4(uint32_t g, uint32_t nib) {
-  const uint32_t x = (nib * 0x00204081u) & 0x01010101u;  // byte j = bit j of the nibble
-  return (g ^ ((x << 8) - x)) + x;
+  const uint32_t x = sign_bits(nib);
+  return (g ^ sign_mask(x)) + x;
 }
 
 // Q8_0: eight blocks of 32 (vec_dot_q8_0_q8_0). Term: the pairwise sum of (d_w d_a) sumi over the eight blocks.
@@ -280,18 +286,18 @@ struct UnitIQ2_S {
 constexpr uint32_t kIq4nlW0 = 0xBFAD9881u, kIq4nlW1 = 0xF6EADDCFu, kIq4nlW2 = 0x26190D01u, kIq4nlW3 = 0x71594535u;
 
 // Four nibbles (the bytes of n, each 0..15) to their four codebook values (signed bytes): two byte permutes pick from
-// table bytes 0-7 and 8-15, bit 3 of each nibble chooses between them.
+// table bytes 0-7 and 8-15, a third chooses between them by bit 3 of each nibble.
 __device__ __forceinline__ uint32_t iq4nl_lookup(uint32_t n) {
   const uint32_t sel = n & 0x07070707u;
   const uint32_t lo = __builtin_amdgcn_perm(kIq4nlW1, kIq4nlW0, sel), hi = __builtin_amdgcn_perm(kIq4nlW3, kIq4nlW2, sel);
-  const uint32_t b = (n >> 3) & 0x01010101u, m = (b << 8) - b;  // 0xff where the nibble is 8..15
-  return (hi & m) | (lo & ~m);
+  // Byte j of hi (permute selector 4 + j) where nibble j is 8..15, else of lo (j).
+  return __builtin_amdgcn_perm(hi, lo, ((n >> 1) & 0x04040404u) | 0x03020100u);
 }
 
 // The four 2-bit codes of byte x (value j at bits 2 j) as four signed bytes q - 1 (Q2_0's -1, 0, 1, 2).
 __device__ __forceinline__ uint32_t q2_spread(uint32_t x) {
   const uint32_t s = (x | (x << 6) | (x << 12) | (x << 18)) & 0x03030303u;
-  return ((s | 0x80808080u) - 0x01010101u) ^ 0x80808080u;  // per byte (0x80 + q) - 1, no borrows, back to q - 1
+  return __builtin_amdgcn_perm(0u, 0x020100ffu, s);  // code q picks byte q of -1, 0, 1, 2
 }
 
 // IQ4_NL: eight blocks of 32, y = d kvalues[nibble] (dequantize_row_iq4_nl; vec_dot_iq4_nl_q8_0 against q8_0). The

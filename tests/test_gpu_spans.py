@@ -1,0 +1,62 @@
+"""The prefill expert GEMMs over spans of one expert's positions (gate/up in two int8 planes, the q8_0 family's down),
+at the edges of their position tiles and spans, against the oracle's compute_many bit for bit; every gate/up and down type
+they take, rows of K that end in a partial unit, and codebooks with too many levels for the planes' digits."""
+import numpy as np
+import pytest
+
+from tests import harness as h
+from tests.harness import moe
+from tests.test_gpu_parity import say
+
+pytestmark = pytest.mark.gpu
+
+# Positions an expert gets: around a position tile (16), a short span (64), a long one (128), and past two of each.
+COUNTS = (1, 15, 16, 17, 63, 64, 65, 128, 129, 257)
+Q8, Q4, I3, NL, XS, Q2, XX, S2 = (moe.QT_Q8_0, moe.QT_Q4_K, moe.QT_IQ3_S, moe.QT_IQ4_NL, moe.QT_IQ4_XS, moe.QT_Q2_0,
+                                  moe.QT_IQ3_XXS, moe.QT_IQ2_S)
+
+
+def check(gt, dt, H, F, codebooks, limit=0.0):
+    E = len(COUNTS)
+    L = h.Layer(H, F, E, E, gt, dt, has_shared=False, seed=910 + gt + F, swiglu_limit=limit)
+    blk = moe.MoeBlock(H, F, E, E, gt, dt, False, max_tokens=260, swiglu_limit=limit)
+    if {gt, dt} & set(moe.CODEBOOK_TYPES):
+        blk.set_codebooks(codebooks)
+    r = np.random.default_rng(5)
+    x = h.tokens(911, 260, H)
+    x[3] = 0.0  # a row whose scale is zero
+    # Each expert's tokens in an order of its own; a token's jobs in expert order.
+    toks = [set(r.permutation(260)[:c].tolist()) for c in COUNTS]
+    jobs = [(L.experts[e], t, float(r.normal())) for t in range(260) for e in range(E) if t in toks[e]]
+    y = blk.compute_many(jobs, x)
+    yo = h.orc_compute_many(gt, dt, H, F, jobs, x, swiglu_limit=limit)
+    blk.close()
+    assert np.array_equal(y, yo), h.max_abs(y, yo)
+
+
+@pytest.mark.parametrize("gt,dt,H,F", [(Q4, NL, 512, 640), (I3, Q2, 512, 320), (XX, NL, 1024, 640), (S2, Q8, 512, 256),
+                                       (XS, NL, 512, 448), (I3, Q4, 2560, 512), (S2, Q2, 2560, 640), (Q8, Q8, 512, 512),
+                                       (Q4, Q8, 512, 960)],
+                         ids=lambda v: moe.TYPE_NAMES.get(v, str(v)))
+def test_spans(gt, dt, H, F):
+    say("spans", (moe.TYPE_NAMES[gt], moe.TYPE_NAMES[dt], H, F))
+    check(gt, dt, H, F, h.CODEBOOKS)
+
+
+def test_spans_swiglu_limit():
+    check(XX, NL, 512, 256, h.CODEBOOKS, limit=0.05)
+
+
+@pytest.mark.parametrize("gt", [XX, S2], ids=lambda v: moe.TYPE_NAMES[v])
+def test_codebooks_past_the_levels(gt):
+    """A caller's tables whose bytes take more values than the planes' digit tables hold run the general path."""
+    book = h.CODEBOOKS.copy()
+    n = 9216 if gt == XX else 8192
+    book[n - 4:n] = (7, 9, 11, 13)
+    try:
+        h.oracle.orc_set_codebooks(h.ptr(book))
+        moe.synth_set_codebooks(book)
+        check(gt, NL, 512, 256, book)
+    finally:
+        h.oracle.orc_set_codebooks(h.ptr(h.CODEBOOKS))
+        moe.synth_set_codebooks(h.CODEBOOKS)
