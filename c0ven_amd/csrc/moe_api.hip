@@ -214,6 +214,9 @@ struct moe_ctx {
   std::vector<const uint8_t *> bc_key;
   std::vector<uint64_t> bc_used;  // the call that last used the slot
   uint64_t bc_calls = 0;
+  uint8_t *stage = nullptr;  // experts in the file's layout on their way into the device layout, then their descriptors
+  uint32_t stage_slots = 0;
+  uint64_t stage_stride = 0;
   uint64_t epoch = 0;          // the last launch's number
   std::vector<std::pair<uint64_t *, uint64_t>> tagged;  // the tagged-record buffers (pointer, records)
   uint32_t grid = 0;           // co-resident work-groups of moe_decode
@@ -474,6 +477,66 @@ void forward_dev(moe_ctx *c, uint32_t layer, const float *x, uint32_t T, float *
   }
   if (c->timing) c->ev_used++;
   if (!direct) copy_routing(ids, w, c->last_ids, c->last_w, T * K, s);
+}
+
+// Experts' bytes go up in the file's layout and are repacked on the device (moe_repack), at most kStageExperts at a time through
+// a staging buffer: their matrices one after another, each 256-byte aligned.
+constexpr uint32_t kStageExperts = 16;
+
+uint64_t file_bytes(uint32_t type, uint64_t rows, uint64_t k) {
+  return (rows * (k / quant_block_values(type)) * quant_block_bytes(type) + 255) / 256 * 256;
+}
+uint64_t stage_bytes(const RepackShape &s) {
+  uint64_t n = 0;
+  for (int m = 0; m < 3; m++) n += file_bytes(s.type[m], s.rows[m], s.cols[m]);
+  return n;
+}
+
+// The staging buffer, for n (at most kStageExperts) experts of the context's largest file layout.
+void stage_experts(moe_ctx *c, uint32_t n) {
+  if (n <= c->stage_slots) return;
+  check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+  const moe_config &g = c->cfg;
+  const auto bytes = [&](uint32_t gt, uint32_t ut, uint32_t dt) {
+    return stage_bytes({{gt, ut, dt}, {g.n_ff, g.n_ff, g.n_embd}, {g.n_embd, g.n_embd, g.n_ff}, {}});
+  };
+  c->stage_stride = std::max(bytes(g.gate_type, g.gate_type, g.down_type),
+                             g.has_shared ? bytes(g.sh_gate_type, g.sh_up_type, g.sh_down_type) : uint64_t(0));
+  void *p = nullptr;
+  check(hipMalloc(&p, n * (c->stage_stride + sizeof(RepackExpert))), "hipMalloc");
+  if (c->stage) {
+    c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void *)c->stage));
+    c->dev_bytes -= c->stage_slots * (c->stage_stride + sizeof(RepackExpert));
+    (void)hipFree(c->stage);
+  }
+  c->allocs.push_back(p);
+  c->stage = (uint8_t *)p, c->stage_slots = n, c->dev_bytes += n * (c->stage_stride + sizeof(RepackExpert));
+}
+
+// Experts ew[0 .. n - 1] (n at most the staging buffer's) into the device layout at dst[i], on a stream, and waits for it.
+void repack_staged(moe_ctx *c, const RepackShape &s, const moe_expert_weights *ew, uint8_t *const *dst, uint32_t n, hipStream_t st) {
+  RepackExpert d[kStageExperts];
+  uint32_t tall = 0;
+  for (uint32_t m = 0; m < 3; m++) tall = std::max(tall, s.rows[m]);
+  for (uint32_t i = 0; i < n; i++) {
+    uint8_t *at = c->stage + i * c->stage_stride;
+    const uint8_t *src[3] = {ew[i].gate, ew[i].up, ew[i].down};
+    for (uint32_t m = 0; m < 3; m++) {
+      const uint64_t row = (uint64_t)(s.cols[m] / quant_block_values(s.type[m])) * quant_block_bytes(s.type[m]);
+      check(hipMemcpyAsync(at, src[m], s.rows[m] * row, hipMemcpyHostToDevice, st), "upload expert");
+      d[i].src[m] = at;
+      at += file_bytes(s.type[m], s.rows[m], s.cols[m]);
+    }
+    d[i].dst = dst[i], d[i].pad = 0;
+    const uint32_t nb = s.cols[2] / quant_block_values(s.type[2]);
+    d[i].down0 = ew[i].down_parts != 2 ? 0u : ew[i].down_blocks[0] ? ew[i].down_blocks[0] : nb / 2;
+  }
+  RepackExpert *dev = (RepackExpert *)(c->stage + c->stage_slots * c->stage_stride);
+  check(hipMemcpyAsync(dev, d, n * sizeof *d, hipMemcpyHostToDevice, st), "upload expert");
+  hipLaunchKernelGGL(moe_repack, dim3((tall + kTileRows - 1) / kTileRows, 3, n), dim3(256), 0, st, (const RepackExpert *)dev, s);
+  check(hipGetLastError(), "moe_repack");
+  // (The descriptors are on this function's stack, and neither they nor the caller's matrices are kept.)
+  check(hipStreamSynchronize(st), "moe_repack");
 }
 
 // A wait inside moe_decode gave up: its result is not to be trusted. The caller has synchronised the stream the
@@ -789,13 +852,12 @@ MOE_API moe_status moe_load_expert(moe_ctx *c, uint32_t layer, uint32_t expert, 
     const uint32_t gt = shared ? g.sh_gate_type : g.gate_type, ut = shared ? g.sh_up_type : g.gate_type;
     const uint32_t dt = shared ? g.sh_down_type : g.down_type;
     const uint64_t gb = matrix_bytes(gt, g.n_ff, g.n_embd), ub = matrix_bytes(ut, g.n_ff, g.n_embd);
-    const uint64_t dn = matrix_bytes(dt, g.n_embd, g.n_ff);
-    std::vector<uint8_t> buf(gb + ub + dn);
-    repack_matrix(gt, gate, g.n_ff, g.n_embd, buf.data());
-    repack_matrix(ut, up, g.n_ff, g.n_embd, buf.data() + gb);
-    repack_matrix(dt, down, g.n_embd, g.n_ff, buf.data() + gb + ub);
     uint8_t *dst = shared ? c->layers[layer].shared : c->layers[layer].experts + (uint64_t)expert * c->ex_bytes;
-    check(hipMemcpy(dst, buf.data(), buf.size(), hipMemcpyHostToDevice), "upload expert");
+    const RepackShape sh{{gt, ut, dt}, {g.n_ff, g.n_ff, g.n_embd}, {g.n_embd, g.n_embd, g.n_ff}, {0, gb, gb + ub}};
+    stage_experts(c, 1);
+    const moe_expert_weights ew{gate, up, down, 1, {0, 0}};
+    // The null stream, as any load: it waits for the work of the blocking streams that may read the old weights.
+    repack_staged(c, sh, &ew, &dst, 1, nullptr);
   });
 }
 
@@ -1037,32 +1099,6 @@ void decode_prerouted(moe_ctx *c, uint32_t layer, const uint8_t *base, const std
   check(hipStreamSynchronize(s), "pre-routed launch");
 }
 
-// One borrowed expert's three matrices (file layout) repacked into the device layout at dst (ex_bytes).
-void repack_borrowed(const moe_ctx *c, const moe_expert_weights &ew, std::vector<uint8_t> &buf,
-                     std::vector<uint8_t> &joined) {
-  const moe_config &g = c->cfg;
-  const uint32_t H = g.n_embd, F = g.n_ff;
-  const uint64_t gu = c->ex_up;
-  buf.resize(c->ex_bytes);
-  repack_matrix(g.gate_type, ew.gate, F, H, buf.data());
-  repack_matrix(g.gate_type, ew.up, F, H, buf.data() + gu);
-  const uint8_t *down = ew.down;
-  if (ew.down_parts == 2) {
-    // The two regions joined row by row into the file's rows: part 0 of every row, then part 1 of every row.
-    const uint64_t bb = quant_block_bytes(g.down_type), bv = quant_block_values(g.down_type);
-    const uint64_t nb = F / bv;
-    const uint64_t b0 = ew.down_blocks[0] ? ew.down_blocks[0] : nb / 2, b1 = ew.down_blocks[0] ? ew.down_blocks[1] : nb - nb / 2;
-    require(b0 + b1 == nb, "down_blocks do not sum to a row");
-    joined.resize(nb * bb * H);
-    for (uint32_t r = 0; r < H; r++) {
-      std::memcpy(joined.data() + r * nb * bb, ew.down + r * b0 * bb, b0 * bb);
-      std::memcpy(joined.data() + r * nb * bb + b0 * bb, ew.down + H * b0 * bb + r * b1 * bb, b1 * bb);
-    }
-    down = joined.data();
-  }
-  repack_matrix(g.down_type, down, H, F, buf.data() + 2 * gu);
-}
-
 MOE_API moe_status moe_compute_many(moe_ctx *c, const moe_cm_job *jobs, uint32_t njobs, uint32_t ntok, const float *x,
                                     uint64_t x_stride, float *y, uint64_t y_stride) {
   return guarded(c, [&] {
@@ -1114,20 +1150,30 @@ MOE_API moe_status moe_compute_many(moe_ctx *c, const moe_cm_job *jobs, uint32_t
       for (uint32_t d = 0; d < nd; d++)
         for (uint32_t sl = 0; sl < c->bc_slots; sl++)
           if (c->bc_key[sl] == dg[d]) slot[d] = sl, c->bc_used[sl] = call;
-    std::vector<uint8_t> buf, joined;
+    std::vector<moe_expert_weights> up;
+    std::vector<uint8_t *> to;
     for (uint32_t d = 0; d < nd; d++) {
       if (slot[d] != UINT32_MAX) continue;
       uint32_t best = 0;  // the least recently used slot this call has not taken
       for (uint32_t sl = 1; sl < c->bc_slots; sl++)
         if (c->bc_used[sl] < c->bc_used[best]) best = sl;
       require(c->bc_used[best] != call, "expert copies exhausted");
-      slot[d] = best, c->bc_used[best] = call, c->bc_key[best] = dg[d];
+      slot[d] = best, c->bc_used[best] = call, c->bc_key[best] = nullptr;
       uint32_t j0 = 0;
       while (dj[j0] != d) j0++;
-      repack_borrowed(c, jobs[j0].expert, buf, joined);
-      check(hipMemcpy(c->bc_base + (uint64_t)best * c->ex_bytes, buf.data(), buf.size(), hipMemcpyHostToDevice),
-            "upload expert");
+      const moe_expert_weights &ew = jobs[j0].expert;
+      require(ew.down_parts == 1 || !ew.down_blocks[0] ||
+                  (uint64_t)ew.down_blocks[0] + ew.down_blocks[1] == F / quant_block_values(g.down_type),
+              "down_blocks do not sum to a row");
+      up.push_back(jobs[j0].expert), to.push_back(c->bc_base + (uint64_t)best * c->ex_bytes);
     }
+    if (!up.empty()) {
+      const RepackShape sh{{g.gate_type, g.gate_type, g.down_type}, {F, F, H}, {H, H, F}, {0, c->ex_up, c->ex_down}};
+      stage_experts(c, std::min<uint32_t>((uint32_t)up.size(), kStageExperts));
+      for (size_t i = 0; i < up.size(); i += c->stage_slots)
+        repack_staged(c, sh, &up[i], &to[i], (uint32_t)std::min<size_t>(c->stage_slots, up.size() - i), c->stream);
+    }
+    for (uint32_t d = 0; d < nd; d++) c->bc_key[slot[d]] = dg[d];
     hipStream_t s = c->stream;
     check(hipMemcpy2DAsync(c->x_dev, H * sizeof(float), x, x_stride * sizeof(float), H * sizeof(float), ntok,
                            hipMemcpyHostToDevice, s),

@@ -4,6 +4,7 @@
 
 #include "aux.h"
 #include "iq3s_grid.h"
+#include "repack.h"
 #include "units.h"
 
 namespace c0ven {
@@ -101,6 +102,43 @@ __global__ void __launch_bounds__(64) moe_dequant(const uint8_t *mat, uint32_t t
         o[i] = __fmul_rn(db, (float)(int8_t)(w.w[i / 4] >> (8 * (i % 4))));
       }
   }
+  }
+}
+
+// File layout to device layout (repack.h's pieces), a row tile of one matrix a work-group: thread e takes piece e / (64 U) of
+// pair e % (64 U), so that a wave's stores are one run of a field. The reads go through L2 (a row tile's file bytes are at most a
+// few hundred KB, each line read by its unit's pieces). What bounds a call is the upload of the same
+// bytes: 4 tokens' borrowed experts of 2560 x 640 (52 MB, IQ3_XXS and IQ4_NL) take 1.86 ms, 7.30 where the host repacked them.
+__global__ void __launch_bounds__(256) moe_repack(const RepackExpert *experts, RepackShape s) {
+  const uint32_t m = blockIdx.y, rt = blockIdx.x, type = s.type[m], k = s.cols[m];
+  if (rt * kTileRows >= s.rows[m]) return;
+  const RepackExpert &ex = experts[blockIdx.z];
+  const uint32_t U = units_of(k), nl = kTileRows * U, bb = quant_block_bytes(type), bv = quant_block_values(type);
+  const uint32_t nb = k / bv, ub = kUnit / bv;  // blocks a row, blocks a unit
+  const uint8_t *src = ex.src[m];
+  const uint32_t b0 = m == 2 && ex.down0 ? ex.down0 : nb;  // blocks a row in the first region
+  uint8_t *tile = ex.dst + s.off[m] + (uint64_t)rt * tile_bytes(type, U);
+  for (uint32_t e = threadIdx.x; e < nl * repack_pieces(type); e += 256) {
+    const uint32_t idx = e % nl, u = idx / kTileRows;
+    const uint64_t row = rt * kTileRows + idx % kTileRows;
+    const RepackPiece p = repack_piece(type, e / nl);
+    const uint32_t blk = u * ub + p.blk;
+    const uint8_t *b = src + (blk < b0 ? (row * b0 + blk) * bb : ((uint64_t)s.rows[m] * b0 + row * (nb - b0) + (blk - b0)) * bb) + p.off;
+    uint8_t *d = tile + (uint64_t)p.field * nl + ((uint64_t)p.piece * nl + idx) * p.stride + p.sub;
+    const bool live = blk < nb;
+    // (The file's blocks are 2-byte aligned, the fields' pieces are aligned to their size.)
+    const auto move = [&](auto v) {
+      if (live) __builtin_memcpy(&v, b, sizeof v);
+      *(decltype(v) *)d = v;
+    };
+    if (p.bytes == 16)
+      move(uint4{0, 0, 0, 0});
+    else if (p.bytes == 8)
+      move(uint2{0, 0});
+    else if (p.bytes == 4)
+      move(0u);
+    else
+      move((uint16_t)0);
   }
 }
 

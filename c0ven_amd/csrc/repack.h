@@ -1,4 +1,5 @@
-// The host's repack of a matrix from the file's layout (ggml blocks, row-major) into the device layout (layout.h).
+// The repack of a matrix from the file's layout (ggml blocks, row-major) into the device layout (layout.h): which bytes go
+// where, for the device's kernel (moe_repack) and the host's form below.
 #pragma once
 
 #include <cstring>
@@ -7,6 +8,53 @@
 #include "layout.h"
 
 namespace c0ven {
+
+// A run of a unit's bytes: bytes (2, 4, 8 or 16) at off of the unit's block blk go to sub of the piece'th stride-byte piece of
+// the field based at field (layout.h), or zeros when the row has no such block.
+struct RepackPiece {
+  uint32_t field, piece, stride, sub, bytes, blk, off;
+};
+C0VEN_HD uint32_t repack_pieces(uint32_t type) {
+  switch (type) {
+    case QT_Q8_0: return 24;
+    case QT_IQ4_NL: return 16;
+    case QT_Q2_0: return 8;
+    case QT_Q4_K: return 12;
+    case QT_IQ3_S: return 10;
+    case QT_IQ3_XXS: return 7;
+    case QT_IQ2_S: return 7;
+    case QT_IQ4_XS: return 9;
+    case QT_Q5_K: return 14;
+    default: return 14;  // QT_Q6_K
+  }
+}
+C0VEN_HD RepackPiece repack_piece(uint32_t type, uint32_t j) {
+  // Piece j of a field of 256-value blocks: n pieces of size bytes from off on.
+  const auto at = [](uint32_t field, uint32_t p, uint32_t size, uint32_t off) { return RepackPiece{field, p, size, 0, size, 0, off + p * size}; };
+  switch (type) {
+    case QT_Q8_0:
+      return j < 16 ? RepackPiece{q8_0t::kQs, j, 16, 0, 16, j / 2, 2 + (j % 2) * 16} : RepackPiece{q8_0t::kD, 0, 16, 2 * (j - 16), 2, j - 16, 0};
+    case QT_IQ4_NL:
+      return j < 8 ? RepackPiece{iq4_nlt::kQs, j, 16, 0, 16, j, 2} : RepackPiece{iq4_nlt::kD, 0, 16, 2 * (j - 8), 2, j - 8, 0};
+    case QT_Q2_0:
+      return j < 4 ? RepackPiece{q2_0t::kQs, j, 16, 0, 16, j, 2} : RepackPiece{q2_0t::kD, 0, 8, 2 * (j - 4), 2, j - 4, 0};
+    case QT_Q4_K: return j < 8 ? at(q4_kt::kQs, j, 16, 16) : j < 11 ? at(q4_kt::kScales, j - 8, 4, 4) : at(q4_kt::kDm, 0, 4, 0);
+    case QT_IQ3_S:
+      return j < 4 ? at(iq3_st::kQs, j, 16, 2) : j < 6 ? at(iq3_st::kSigns, j - 4, 16, 74) : j < 8 ? at(iq3_st::kQh, j - 6, 4, 66)
+             : j < 9 ? at(iq3_st::kScales, 0, 4, 106) : at(iq3_st::kD, 0, 2, 0);
+    case QT_IQ3_XXS: return j < 4 ? at(iq3_xxst::kQs, j, 16, 2) : j < 6 ? at(iq3_xxst::kSs, j - 4, 16, 66) : at(iq3_xxst::kD, 0, 2, 0);
+    case QT_IQ2_S:
+      return j < 2 ? at(iq2_st::kQs, j, 16, 2) : j < 4 ? at(iq2_st::kSigns, j - 2, 16, 34) : j < 5 ? at(iq2_st::kQh, 0, 8, 66)
+             : j < 6 ? at(iq2_st::kScales, 0, 8, 74) : at(iq2_st::kD, 0, 2, 0);
+    case QT_IQ4_XS: return j < 8 ? at(iq4_xst::kQs, j, 16, 8) : at(iq4_xst::kMeta, 0, 8, 0);
+    case QT_Q5_K:
+      return j < 8 ? at(q5_kt::kQs, j, 16, 48) : j < 10 ? at(q5_kt::kQh, j - 8, 16, 16) : j < 13 ? at(q5_kt::kScales, j - 10, 4, 4)
+             : at(q5_kt::kDm, 0, 4, 0);
+    default:  // QT_Q6_K
+      return j < 8 ? at(q6_kt::kQl, j, 16, 0) : j < 12 ? at(q6_kt::kQh, j - 8, 16, 128) : j < 13 ? at(q6_kt::kScales, 0, 16, 192)
+             : at(q6_kt::kD, 0, 2, 208);
+  }
+}
 
 // Row r's unit u in the file's layout: the bytes of its blocks (Q8_0: 8 blocks of 34 B; IQ4_NL: 8 of 18 B; Q2_0: 4
 // of 18 B; the 256-value types: one block).
@@ -17,60 +65,10 @@ inline const uint8_t *file_unit(const uint8_t *m, uint32_t type, uint32_t k, uin
 
 // One unit's bytes into pair idx of a tile of nl = 64 U pairs.
 inline void put_unit(uint8_t *tile, uint32_t type, uint32_t idx, uint32_t nl, const uint8_t *b) {
-  auto at = [&](uint32_t base, uint32_t p, uint32_t piece) { return tile + (uint64_t)base * nl + ((uint64_t)p * nl + idx) * piece; };
-  switch (type) {
-    case QT_Q8_0:
-      for (uint32_t p = 0; p < 16; p++) std::memcpy(at(q8_0t::kQs, p, 16), b + (p / 2) * 34 + 2 + (p % 2) * 16, 16);
-      for (uint32_t blk = 0; blk < 8; blk++) std::memcpy(at(q8_0t::kD, 0, 16) + 2 * blk, b + blk * 34, 2);
-      break;
-    case QT_Q4_K:
-      for (uint32_t p = 0; p < 8; p++) std::memcpy(at(q4_kt::kQs, p, 16), b + 16 + 16 * p, 16);
-      for (uint32_t i = 0; i < 3; i++) std::memcpy(at(q4_kt::kScales, i, 4), b + 4 + 4 * i, 4);
-      std::memcpy(at(q4_kt::kDm, 0, 4), b, 4);
-      break;
-    case QT_IQ4_NL:
-      for (uint32_t p = 0; p < 8; p++) std::memcpy(at(iq4_nlt::kQs, p, 16), b + 18 * p + 2, 16);
-      for (uint32_t blk = 0; blk < 8; blk++) std::memcpy(at(iq4_nlt::kD, 0, 16) + 2 * blk, b + 18 * blk, 2);
-      break;
-    case QT_Q2_0:
-      for (uint32_t p = 0; p < 4; p++) std::memcpy(at(q2_0t::kQs, p, 16), b + 18 * p + 2, 16);
-      for (uint32_t blk = 0; blk < 4; blk++) std::memcpy(at(q2_0t::kD, 0, 8) + 2 * blk, b + 18 * blk, 2);
-      break;
-    case QT_IQ3_XXS:
-      for (uint32_t p = 0; p < 4; p++) std::memcpy(at(iq3_xxst::kQs, p, 16), b + 2 + 16 * p, 16);
-      for (uint32_t p = 0; p < 2; p++) std::memcpy(at(iq3_xxst::kSs, p, 16), b + 66 + 16 * p, 16);
-      std::memcpy(at(iq3_xxst::kD, 0, 2), b, 2);
-      break;
-    case QT_IQ2_S:
-      for (uint32_t p = 0; p < 2; p++) std::memcpy(at(iq2_st::kQs, p, 16), b + 2 + 16 * p, 16);
-      for (uint32_t p = 0; p < 2; p++) std::memcpy(at(iq2_st::kSigns, p, 16), b + 34 + 16 * p, 16);
-      std::memcpy(at(iq2_st::kQh, 0, 8), b + 66, 8);
-      std::memcpy(at(iq2_st::kScales, 0, 8), b + 74, 8);
-      std::memcpy(at(iq2_st::kD, 0, 2), b, 2);
-      break;
-    case QT_IQ4_XS:
-      for (uint32_t p = 0; p < 8; p++) std::memcpy(at(iq4_xst::kQs, p, 16), b + 8 + 16 * p, 16);
-      std::memcpy(at(iq4_xst::kMeta, 0, 8), b, 8);
-      break;
-    case QT_Q5_K:
-      for (uint32_t p = 0; p < 8; p++) std::memcpy(at(q5_kt::kQs, p, 16), b + 48 + 16 * p, 16);
-      for (uint32_t p = 0; p < 2; p++) std::memcpy(at(q5_kt::kQh, p, 16), b + 16 + 16 * p, 16);
-      for (uint32_t i = 0; i < 3; i++) std::memcpy(at(q5_kt::kScales, i, 4), b + 4 + 4 * i, 4);
-      std::memcpy(at(q5_kt::kDm, 0, 4), b, 4);
-      break;
-    case QT_Q6_K:
-      for (uint32_t p = 0; p < 8; p++) std::memcpy(at(q6_kt::kQl, p, 16), b + 16 * p, 16);
-      for (uint32_t p = 0; p < 4; p++) std::memcpy(at(q6_kt::kQh, p, 16), b + 128 + 16 * p, 16);
-      std::memcpy(at(q6_kt::kScales, 0, 16), b + 192, 16);
-      std::memcpy(at(q6_kt::kD, 0, 2), b + 208, 2);
-      break;
-    case QT_IQ3_S:
-      for (uint32_t p = 0; p < 4; p++) std::memcpy(at(iq3_st::kQs, p, 16), b + 2 + 16 * p, 16);
-      for (uint32_t p = 0; p < 2; p++) std::memcpy(at(iq3_st::kSigns, p, 16), b + 74 + 16 * p, 16);
-      for (uint32_t i = 0; i < 2; i++) std::memcpy(at(iq3_st::kQh, i, 4), b + 66 + 4 * i, 4);
-      std::memcpy(at(iq3_st::kScales, 0, 4), b + 106, 4);
-      std::memcpy(at(iq3_st::kD, 0, 2), b, 2);
-      break;
+  const uint32_t bb = quant_block_bytes(type);
+  for (uint32_t j = 0; j < repack_pieces(type); j++) {
+    const RepackPiece p = repack_piece(type, j);
+    std::memcpy(tile + (uint64_t)p.field * nl + ((uint64_t)p.piece * nl + idx) * p.stride + p.sub, b + p.blk * bb + p.off, p.bytes);
   }
 }
 
