@@ -56,6 +56,8 @@ struct Layer {
   float *hc_gamma = nullptr;
   uint16_t *hc_down = nullptr, *hc_inj = nullptr, *hc_up = nullptr;
   double *hc_rn = nullptr;  // the 2-norms of W_down's, W_inject's and W_up's rows (the prefill mix's bound)
+  uint8_t *hc_dig_down = nullptr, *hc_dig_up = nullptr;  // the digits of W_down's and W_inject's rows, of W_up's (prefill)
+  HcGrid hc_grid{};         // their grids
   int *hc_rlsb = nullptr;   // the least lsb exponent of each of those rows' nonzero bf16 values
   bool has_hc = false;
 };
@@ -637,6 +639,12 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
         L.hc_up = c->alloc<uint16_t>((uint64_t)kHcStreams * H * g.hc_lr);
         L.hc_rn = c->alloc<double>((uint64_t)g.hc_lr + kHcStreams + (uint64_t)kHcStreams * H);
         L.hc_rlsb = c->alloc<int>((uint64_t)g.hc_lr + kHcStreams + (uint64_t)kHcStreams * H);
+        if (g.max_tokens > kMaxDecodeTokens) {
+          L.hc_dig_down = c->alloc<uint8_t>(hc_digit_bytes((uint64_t)g.hc_lr + kHcStreams, (uint64_t)kHcStreams * H));
+          L.hc_dig_up = c->alloc<uint8_t>(hc_digit_bytes((uint64_t)kHcStreams * H, g.hc_lr));
+          L.hc_grid.exp = c->alloc<int>((uint64_t)g.hc_lr + kHcStreams + (uint64_t)kHcStreams * H);
+          L.hc_grid.lost = c->alloc<uint32_t>((uint64_t)g.hc_lr + kHcStreams + (uint64_t)kHcStreams * H);
+        }
       }
     }
     // Scratch for max_tokens tokens of n_used + 1 assignments (the pre-routed path may give a token its shared
@@ -735,6 +743,9 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
         b.cnt = c->alloc<uint32_t>(2);
         b.lb = c->alloc<uint16_t>(TM * g.hc_lr);
         b.nb = c->alloc<uint16_t>(TM * D);
+        b.nd = c->alloc<uint8_t>(hc_digit_bytes(TM, D));
+        b.ld = c->alloc<uint8_t>(hc_digit_bytes(TM, g.hc_lr));
+        for (HcGrid *q : {&b.ng, &b.lg}) q->exp = c->alloc<int>(TM), q->lost = c->alloc<uint32_t>(TM);
         b.ln = c->alloc<double>(TM);
         b.inj = c->alloc<float>(TM * kHcStreams);
         b.a = c->alloc<float>(TM * D);
@@ -932,6 +943,10 @@ MOE_API moe_status moe_forward_async(moe_ctx *c, uint32_t layer, const float *x_
   });
 }
 
+HcLayer hc_layer(const Layer &L) {
+  return {L.hc_gamma, L.hc_down, L.hc_inj, L.hc_up, L.hc_rn, L.hc_rlsb, L.hc_dig_down, L.hc_dig_up, L.hc_grid};
+}
+
 MOE_API moe_status moe_load_hc(moe_ctx *c, uint32_t layer, const float *gamma, const uint16_t *w_down,
                                const uint16_t *w_inject, const uint16_t *w_up) {
   return guarded(c, [&] {
@@ -963,13 +978,22 @@ MOE_API moe_status moe_load_hc(moe_ctx *c, uint32_t layer, const float *gamma, c
         if (w[i] & 0x7fffu) m = std::min(m, ((w[i] >> 7) & 0xffu) == 0u ? -133 : (int)((w[i] >> 7) & 0xffu) - 134);
       return m;
     };
-    for (uint32_t j = 0; j < g.hc_lr; j++) rn[j] = norm(w_down + (uint64_t)j * D, D), rl[j] = lsb(w_down + (uint64_t)j * D, D);
-    for (uint32_t j = 0; j < kHcStreams; j++)
-      rn[g.hc_lr + j] = norm(w_inject + (uint64_t)j * D, D), rl[g.hc_lr + j] = lsb(w_inject + (uint64_t)j * D, D);
-    for (uint64_t j = 0; j < D; j++)
-      rn[g.hc_lr + kHcStreams + j] = norm(w_up + j * g.hc_lr, g.hc_lr), rl[g.hc_lr + kHcStreams + j] = lsb(w_up + j * g.hc_lr, g.hc_lr);
+    std::vector<int> re(rn.size());  // the largest exponent fields
+    const auto row = [&](uint64_t j, const uint16_t *w, uint64_t n) {
+      rn[j] = norm(w, n), rl[j] = lsb(w, n), re[j] = 0;
+      for (uint64_t i = 0; i < n; i++) re[j] = std::max(re[j], (int)((w[i] >> 7) & 0xffu));
+    };
+    for (uint32_t j = 0; j < g.hc_lr; j++) row(j, w_down + (uint64_t)j * D, D);
+    for (uint32_t j = 0; j < kHcStreams; j++) row(g.hc_lr + j, w_inject + (uint64_t)j * D, D);
+    for (uint64_t j = 0; j < D; j++) row(g.hc_lr + kHcStreams + j, w_up + j * g.hc_lr, g.hc_lr);
     check(hipMemcpy(L.hc_rn, rn.data(), rn.size() * sizeof(double), hipMemcpyHostToDevice), "upload hc norms");
     check(hipMemcpy(L.hc_rlsb, rl.data(), rl.size() * sizeof(int), hipMemcpyHostToDevice), "upload hc lsb");
+    if (L.hc_dig_down) {  // the digits, on the null stream like the copies
+      check(hipMemcpy(L.hc_grid.exp, re.data(), re.size() * sizeof(int), hipMemcpyHostToDevice), "upload hc exponents");
+      check(hipMemset(L.hc_grid.lost, 0, re.size() * sizeof(uint32_t)), "hipMemset");
+      check(prefill_hc_load(g.n_embd, g.hc_lr, hc_layer(L), L.hc_dig_down, L.hc_dig_up, nullptr), "hc digits launch");
+      check(hipStreamSynchronize(nullptr), "hc digits");
+    }
     L.has_hc = true;
   });
 }
@@ -989,8 +1013,7 @@ MOE_API moe_status moe_forward_hc_async(moe_ctx *c, uint32_t layer, float *R_dev
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     if (ntok > c->tdec) {  // the prefill path: the mix's kernels, the block, the combine's kernel
       const HcShape S{g.n_embd, g.hc_lr, ntok};
-      const HcLayer HL{L.hc_gamma, L.hc_down, L.hc_inj, L.hc_up, L.hc_rn, L.hc_rlsb};
-      check(prefill_hc_pre(S, HL, c->hcp, R_dev, (g.flags & MOE_FLAG_HC_FIXED_ORDER) != 0, s), "prefill hc mix launch");
+      check(prefill_hc_pre(S, hc_layer(L), c->hcp, R_dev, (g.flags & MOE_FLAG_HC_FIXED_ORDER) != 0, s), "prefill hc mix launch");
       float *y = y_dev ? y_dev : c->y_dev;
       forward_dev(c, layer, c->hcp.x, ntok, y, ids_dev, w_dev, s);
       check(prefill_hc_post(S, c->hcp, R_dev, y, s), "prefill hc combine launch");

@@ -4,13 +4,14 @@
 // The results are the decode path's, bit for bit (and the oracle's, orc_hc_pre / orc_hc_post): the norms, silu,
 // sigmoid and mix steps are the same fp32 operations; the two bf16 products (W_down and W_inject against n, W_up
 // against l) are sums of exact products that the decode kernel adds in fp64 in a fixed order and rounds to fp32 once.
-// Here they run on the fp64 matrix cores (v_mfma_f64_16x16x4f64) in another order, with a bound on the difference:
-// each sum path has at most n_mine roundings here and n_ref in the fixed order, so the two fp64 values are within
-// (n_mine + n_ref) 2^-53 sum|p| <= (n_mine + n_ref) 2^-53 ||w||_2 ||x||_2 of each other (Cauchy-Schwarz on the bf16
-// values). Where the fp32 rounding of every value in that interval is the same, it is the fixed order's rounding; and
-// where the products' bits span fewer than 53 (the least lsb of the row's and of the token's values against the
-// Cauchy-Schwarz bound on sum|p|), both sums are exact, whatever their order (ties of fp32 rounding are common for
-// W_up's short sums, and this settles them).
+// Here they run on the int8 matrix cores: a row's or token's bf16 values become whole numbers of 2^-29 of its largest
+// value's power of two, in four signed byte digits, and the digits' products add exactly in 32 bits (a value more than
+// 2^22 below the largest loses bits; those are counted). The exact sum, rounded once a K part, is then within
+// (n_mine + n_ref) 2^-53 sum|p| <= (n_mine + n_ref) 2^-53 ||w||_2 ||x||_2 of the fixed order's (Cauchy-Schwarz on the
+// bf16 values; the lost bits add their own term). Where the fp32 rounding of every value in that interval is the same,
+// it is the fixed order's rounding; and where the products' bits span fewer than 53 (the least lsb of the row's and of
+// the token's values against the Cauchy-Schwarz bound on sum|p|), both sums are exact, whatever their order (ties of
+// fp32 rounding are common for W_up's short sums, and this settles them).
 // Otherwise the sum is recomputed in the fixed order, one wave an open sum, from a list, in a kernel of its own:
 // W_up's a k-order chain of at most 512 terms, W_down's and W_inject's the decode kernel's 512-value-chunk tree.
 #include <hip/hip_runtime.h>
@@ -21,11 +22,11 @@
 namespace c0ven {
 namespace {
 
-typedef double v4d_t __attribute__((ext_vector_type(4)));
+typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kHcWG = 256;
 constexpr uint32_t kHcStreams4 = 4;
-constexpr uint32_t kGroupK = 128;  // values a matrix-core chain sums before its sum joins the fp64 total
+constexpr uint32_t kDiagonals = 2 * kHcDigits - 1;  // the digit products' weights: 256^0 .. 256^6
 
 __device__ __forceinline__ uint32_t lane_of() { return threadIdx.x & 63u; }
 
@@ -64,15 +65,18 @@ __device__ __forceinline__ int wg_min(int v, int *red) {
 
 // Token t (one work-group): each stream as RMSNorm(R_s) gamma_s, the decode kernel's hc_norm_item arithmetic (each
 // thread's squares in order, then wg_sum; mean rounded to fp32; 1 / sqrtf(mean + 1e-6)): the stream's scale into sc
-// (pf_hc_mix forms n again from R, the scale and gamma), bf16(n) into nb, and the 2-norm (rounded up) and least lsb
-// exponent of bf16(n). Work-group 0 clears the open lists' counts.
+// (pf_hc_mix forms n again from R, the scale and gamma), bf16(n) into nb, and the 2-norm (rounded up), least lsb
+// exponent and largest exponent field of bf16(n). Work-group 0 clears the open lists' counts, each its token's counts of
+// values that lose bits.
 __global__ void __launch_bounds__(kHcWG) pf_hc_norm(const float *R, const float *gamma, uint32_t H, float *sc,
-                                                    uint16_t *nb, double *nn, int *nlsb, uint32_t *cnt) {
+                                                    uint16_t *nb, double *nn, int *nlsb, HcGrid n, HcGrid l,
+                                                    uint32_t *cnt) {
   __shared__ double red[4];
   __shared__ int redi[4];
-  int lsb = 1 << 20;
+  int lsb = 1 << 20, top = 0;
   const uint32_t t = blockIdx.x;
   if (t == 0 && threadIdx.x < 2) cnt[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) n.lost[t] = l.lost[t] = 0u;
   double sq = 0.0;
   for (uint32_t s = 0; s < kHcStreams4; s++) {
     const float *r = R + ((uint64_t)t * kHcStreams4 + s) * H;
@@ -90,123 +94,227 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_norm(const float *R, const float 
       const double b = (double)bv;
       sq = __builtin_fma(b, b, sq);
       lsb = min(lsb, bf16_lsb_of(bv));
+      top = max(top, (int)((__float_as_uint(bv) >> 23) & 0xffu));
     }
   }
   sq = wg_sum(sq, red);
   lsb = wg_min(lsb, redi);
+  top = -wg_min(-top, redi);
+  if (threadIdx.x == 0) n.exp[t] = top;
   if (threadIdx.x == 0) nn[t] = sqrt(sq) * (1.0 + 0x1p-30), nlsb[t] = lsb;
 }
 
-// Whether an fp64 sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: every
-// product is a multiple of 2^(lr + lt) and sum|p| <= rn tn < 2^(lr + lt + 53), so every partial sum of any order is
-// representable and both orders give the exact sum. Otherwise bounded: the two fp64 values are within bnd, and every
-// value in [v - bnd, v + bnd] rounds to the same fp32.
-__device__ __forceinline__ bool certain(double v, double rn, double tn, int lr, int lt, double bound_k) {
+// Four values' digits (X as bytes after the carry trick below) as four words of one digit each.
+__device__ __forceinline__ void transpose4(const uint32_t y[4], uint32_t d[kHcDigits]) {
+  const uint32_t a0 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), a1 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
+  const uint32_t b0 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u), b1 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+  d[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100u), d[1] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+  d[2] = __builtin_amdgcn_perm(b1, a1, 0x05040100u), d[3] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+}
+
+// The digits of bf16 rows (A0's first M0, then A1's; K values each, a multiple of 8) whose largest exponent fields are
+// g.exp: value (-1)^s m 2^(e - 134) is the whole number X = (-1)^s m 2^(e - exp + 22), toward zero (|X| < 2^30), and
+// X = sum of d_i 256^i with d_i in -128 .. 127. The rows are laid out as the matrix cores take them: 16-row tile, 64
+// values, digit, then lane 16 q + r's 16 values 16 q .. of row r; rows and values past the ends are zeros. A wave a tile's
+// 64 values: it reads 128 bytes of each row and writes 4 KB whole. g.lost[row] counts the values that lost bits.
+__global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32_t M0, const uint16_t *A1, uint32_t M,
+                                                      uint32_t K, HcGrid g, uint8_t *out) {
+  const uint32_t nch = (K + 63) / 64, ch = blockIdx.y * (kHcWG / 64) + (threadIdx.x >> 6);
+  if (ch >= nch) return;
+  const uint32_t lane = lane_of(), row = 16 * blockIdx.x + lane % 16, k0 = 64 * ch + 16 * (lane / 16);
+  uint32_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  int top = 0;
+  if (row < M) {
+    const uint16_t *src = (row < M0 ? A0 + (uint64_t)row * K : A1 + (uint64_t)(row - M0) * K) + k0;
+    top = g.exp[row];
+    if (k0 < K) {
+      const uint4 q = *(const uint4 *)src;
+      v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+    }
+    if (k0 + 8 < K) {
+      const uint4 q = *(const uint4 *)(src + 8);
+      v[4] = q.x, v[5] = q.y, v[6] = q.z, v[7] = q.w;
+    }
+  }
+  uint32_t lost = 0, d[4][kHcDigits];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    uint32_t y[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t u = (v[2 * q + i / 2] >> (16 * (i & 1))) & 0xffffu, e = (u >> 7) & 0xffu;
+      const uint32_t m = (u & 0x7fu) | (e ? 0x80u : 0u);
+      const int sh = (int)max(e, 1u) - max(top, 1) + 22;  // (at most 22)
+      const uint32_t down = (uint32_t)min(max(-sh, 0), 31);
+      const uint32_t x = sh >= 0 ? m << sh : m >> down;
+      lost += (x << down) != m && sh < 0;
+      const uint32_t X = (u & 0x8000u) ? 0u - x : x;
+      y[i] = (X + 0x00808080u) ^ 0x00808080u;  // each lower byte's digit as a signed byte, its carry in the next
+    }
+    transpose4(y, d[q]);
+  }
+  if (lost) atomicAdd(g.lost + row, lost);
+  uint8_t *o = out + ((uint64_t)blockIdx.x * nch + ch) * (kHcDigits * 1024) + lane * 16;
+#pragma unroll
+  for (uint32_t i = 0; i < kHcDigits; i++) *(uint4 *)(o + 1024 * i) = make_uint4(d[0][i], d[1][i], d[2][i], d[3][i]);
+}
+
+// A row's or token's part of the bound: 2-norm (rounded up), least lsb exponent, and the 2-norm of its lost bits (each
+// less than one of its grid's units, 2^(exp - 156); 0: none).
+struct Side {
+  double norm, lost;
+  int lsb, exp;
+};
+__device__ __forceinline__ Side side_of(const double *norm, const int *lsb, const HcGrid &g, uint32_t i) {
+  const uint32_t n = g.lost[i];
+  const int e = max(g.exp[i], 1);
+  return {norm[i], n ? ldexp(sqrt((double)n) * 1.0001, e - 156) : 0.0, lsb[i], e};
+}
+
+// Whether the digits' sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: no
+// bits lost, every product is a multiple of 2^(r.lsb + t.lsb) and sum|p| <= r.norm t.norm < 2^(r.lsb + t.lsb + 53), so
+// every partial sum of any order is representable and both give the exact sum. Otherwise bounded: the two fp64 values
+// are within bnd, and every value in [v - bnd, v + bnd] rounds to the same fp32.
+__device__ __forceinline__ bool certain(double v, const Side &r, const Side &t, double bound_k) {
   if (!__builtin_isfinite(v)) return false;
-  const double m = rn * tn;
-  if (lr + lt < 900 && m < ldexp(1.0, lr + lt + 53)) return true;
-  const double bnd = bound_k * m;
+  const double m = r.norm * t.norm, lost = r.lost * t.norm + r.norm * t.lost;
+  if (lost == 0.0 && r.lsb + t.lsb < 900 && m < ldexp(1.0, r.lsb + t.lsb + 53)) return true;
+  const double bnd = bound_k * m + lost;
   const float f = (float)v;
   return (float)(v - bnd) == f && (float)(v + bnd) == f;
 }
 
-// C = A B^T on the fp64 matrix cores, both bf16: rows of A (M of them: A0's first M0, then A1's), tokens of B (N rows
-// of K), K values. A work-group takes 64 rows x 64 tokens over the K range of its split
-// (blockIdx.y), wave w rows 32 (w & 1) .. and tokens 32 (w >> 1) .., as 2 x 2 tiles of 16 x 16. Lane l (g = l / 16)
-// holds A[row l % 16][k + 4 g + m] and B[token l % 16][k + 4 g + m] for MFMA step m of a 16-value chunk: both operands
-// take the same k in the same place, so each step adds 64 of the row-token products (the order of a sum is free
-// here: the bound covers any). Each kGroupK values' chain starts from zero and is added to an fp64 total.
-// kUp: one split; the sums are certified here (row norms rn, token norms tn) and written as fp32 to out32 (N x M), an
-// open one's (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the fp64 totals go to part
-// (split x N x M).
+// sum of s[i] 256^i, rounded to fp64 once: the low three and the high four weights as 64-bit integers, then 2^40 h + l
+// with both parts exact in fp64.
+__device__ __forceinline__ double diagonals(const int s[kDiagonals]) {
+  const int64_t lo = (int64_t)s[0] + ((int64_t)s[1] << 8) + ((int64_t)s[2] << 16);
+  const int64_t hi = (int64_t)s[3] + ((int64_t)s[4] << 8) + ((int64_t)s[5] << 16) + ((int64_t)s[6] << 24) + (lo >> 24);
+  const uint64_t l40 = ((uint64_t)(hi & 0xffff) << 24) | (uint64_t)(lo & 0xffffff);
+  return __builtin_fma((double)(hi >> 16), 0x1p40, (double)l40);
+}
+
+// C = A B^T over the digits of the rows (M of them, A) and of the tokens (N, B), nch 64-value chunks in blockIdx.x % nsplit
+// parts of cs. A work-group takes 64 rows x 64 tokens, wave w rows 32 (w & 1) .. and tokens 32 (w >> 1) .., as 2 x 2 tiles
+// of 16 x 16, whose digit products of one weight share an accumulator (a part has at most 4096 values: 2^28).
+// The lowest digit is nonzero only for values 2^15 and more below their row's largest (about one in 5000 of a normal
+// row's): a fragment whose lowest digits are all zero skips its products, which leaves 9 of 16 in most chunks.
+// The operands come straight from L2 in the matrix cores' order, the next chunk's while this one's products run.
+// A part keeps to one XCD (nsplit 8), so that each L2 reads one part of both operands; without parts the XCD
+// takes every eighth row tile.
+// kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
+// (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M).
+// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 52 us and up 65, where the fp64 matrix cores took 162 and 141.
 template <bool kUp>
-__global__ void __launch_bounds__(kHcWG) pf_hc_gemm(const uint16_t *A0, uint32_t M0, const uint16_t *A1, uint32_t M,
-                                                    uint32_t K, const uint16_t *B, uint32_t N, uint32_t ksplit,
-                                                    double *part, float *out32, const double *rn, const double *tn,
-                                                    const int *rl, const int *tl, double bound_k, uint32_t *open,
-                                                    uint32_t *cnt) {
-  const uint32_t nmt = (M + 63) / 64, mt = blockIdx.x % nmt, nt = blockIdx.x / nmt, split = blockIdx.y;
+__global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
+                                                       uint32_t nch, uint32_t nsplit, double *part, float *out32,
+                                                       const double *rn, const double *tn, const int *rl,
+                                                       const int *tl, HcGrid gr, HcGrid gt, double bound_k,
+                                                       uint32_t *open, uint32_t *cnt) {
+  const uint32_t nmt = (M + 63) / 64, split = blockIdx.x % nsplit, item = blockIdx.x / nsplit;
+  const uint32_t mt = item % nmt, nt = item / nmt, cs = nch / nsplit;
   const uint32_t lane = lane_of(), w = threadIdx.x >> 6, g = lane / 16, c16 = lane % 16;
   const uint32_t m0 = 64 * mt + 32 * (w & 1), n0 = 64 * nt + 32 * (w >> 1);
-  // 16 x 16 tiles wholly past the rows or the tokens (the down GEMM's last row tile holds 4 of W_inject's rows) are
-  // skipped: a wave with none returns (the kernel has no barrier), the others skip the MFMAs of theirs.
+  // 16 x 16 tiles wholly past the rows or the tokens are skipped: a wave with none returns (the kernel has no barrier),
+  // the others repeat their first tile's operands and drop its sums.
   if (m0 >= M || n0 >= N) return;
-  const bool live_i1 = m0 + 16 < M, live_j1 = n0 + 16 < N;
-  const uint16_t *ar[2];
-  const uint16_t *br[2];
-#pragma unroll
-  for (int f = 0; f < 2; f++) {
-    const uint32_t row = min(m0 + 16 * f + c16, M - 1), tok = min(n0 + 16 * f + c16, N - 1);
-    ar[f] = row < M0 ? A0 + (uint64_t)row * K : A1 + (uint64_t)(row - M0) * K;
-    br[f] = B + (uint64_t)tok * K;
-  }
-  const uint32_t kb = split * ksplit, ke = min(K, kb + ksplit);
-  v4d_t tot[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) tot[i][j] = v4d_t{0.0, 0.0, 0.0, 0.0};
-  for (uint32_t kg = kb; kg < ke; kg += kGroupK) {
-    v4d_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = v4d_t{0.0, 0.0, 0.0, 0.0};
-    const uint32_t kge = min(ke, kg + kGroupK);
-#pragma unroll 2
-    for (uint32_t kc = kg; kc < kge; kc += 16) {
-      const uint32_t k = kc + 4 * g;
-      const bool ok = k < kge;  // (K is a multiple of 4: a lane's four values are all in or all out)
-      uint2 a[2], b[2];
-#pragma unroll
-      for (int f = 0; f < 2; f++) {
-        a[f] = ok ? *(const uint2 *)(ar[f] + k) : make_uint2(0u, 0u);
-        b[f] = ok ? *(const uint2 *)(br[f] + k) : make_uint2(0u, 0u);
-      }
-      double ad[2][4], bd[2][4];
-#pragma unroll
-      for (int f = 0; f < 2; f++) {
-        ad[f][0] = bf16_lo(a[f].x), ad[f][1] = bf16_hi(a[f].x), ad[f][2] = bf16_lo(a[f].y), ad[f][3] = bf16_hi(a[f].y);
-        bd[f][0] = bf16_lo(b[f].x), bd[f][1] = bf16_hi(b[f].x), bd[f][2] = bf16_lo(b[f].y), bd[f][3] = bf16_hi(b[f].y);
-      }
-#pragma unroll
-      for (int m = 0; m < 4; m++)
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < 2; j++)
-          if ((i == 0 || live_i1) && (j == 0 || live_j1))
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[i][m], bd[j][m], acc[i][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) tot[i][j][q] = __dadd_rn(tot[i][j][q], acc[i][j][q]);
-  }
-  // tot[i][j][q]: row m0 + 16 i + 4 q + g, token n0 + 16 j + c16 (the f64 form's result layout: element q of lane l
-  // is row 4 q + l / 16).
+  const uint32_t i1 = m0 + 16 < M ? 1u : 0u, j1 = n0 + 16 < N ? 1u : 0u;
+  const uint64_t tile = (uint64_t)nch * (kHcDigits * 1024), first = (uint64_t)split * cs * (kHcDigits * 1024) + lane * 16;
+  const uint8_t *ap[2] = {A + m0 / 16 * tile + first, A + (m0 / 16 + i1) * tile + first};
+  const uint8_t *bp[2] = {B + n0 / 16 * tile + first, B + (n0 / 16 + j1) * tile + first};
+  v4i_t acc[2][2][kDiagonals];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
+      for (uint32_t d = 0; d < kDiagonals; d++) acc[i][j][d] = v4i_t{0, 0, 0, 0};
+  v4i_t a[2][kHcDigits], b[2][kHcDigits];
+  const auto load = [&](uint32_t c, v4i_t (&to)[2][kHcDigits], const uint8_t *const (&from)[2]) {
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (uint32_t d = 0; d < kHcDigits; d++) to[f][d] = *(const v4i_t *)(from[f] + (c * kHcDigits + d) * 1024);
+  };
+  load(0, a, ap), load(0, b, bp);
+  for (uint32_t c = 0; c < cs; c++) {
+    v4i_t na[2][kHcDigits], nb[2][kHcDigits];
+    const uint32_t next = min(c + 1, cs - 1);
+    load(next, na, ap), load(next, nb, bp);
+#pragma unroll
+    for (uint32_t da = 1; da < kHcDigits; da++)
+#pragma unroll
+      for (uint32_t db = 1; db < kHcDigits; db++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            acc[i][j][da + db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][da], b[j][db], acc[i][j][da + db], 0, 0, 0);
+    const auto any = [](const v4i_t &v) { return __any((v[0] | v[1] | v[2] | v[3]) != 0) != 0; };
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      if (any(a[i][0]))
+#pragma unroll
+        for (uint32_t db = 0; db < kHcDigits; db++)
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            acc[i][j][db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][0], b[j][db], acc[i][j][db], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+      if (any(b[j][0]))
+#pragma unroll
+        for (uint32_t da = 1; da < kHcDigits; da++)
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+            acc[i][j][da] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][da], b[j][0], acc[i][j][da], 0, 0, 0);
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (uint32_t d = 0; d < kHcDigits; d++) a[f][d] = na[f][d], b[f][d] = nb[f][d];
+  }
+  // acc[i][j][.][q]: row m0 + 16 i + 4 g + q, token n0 + 16 j + c16. (M is a multiple of 4.)
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t row = m0 + 16 * i + 4 * g;
+    if (row >= M) continue;
+    Side rs[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if constexpr (kUp)
+        rs[q] = side_of(rn, rl, gr, row + q);
+      else
+        rs[q].exp = max(gr.exp[row + q], 1);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const uint32_t tok = n0 + 16 * j + c16;
+      if (tok >= N) continue;
+      Side ts;
+      if constexpr (kUp)
+        ts = side_of(tn, tl, gt, tok);
+      else
+        ts.exp = max(gt.exp[tok], 1);
+      double v[4];
+#pragma unroll
       for (int q = 0; q < 4; q++) {
-        const uint32_t row = m0 + 16 * i + 4 * q + g, tok = n0 + 16 * j + c16;
-        if (row >= M || tok >= N) continue;
-        const double v = tot[i][j][q];
-        if constexpr (kUp) {
-          if (certain(v, rn[row], tn[tok], rl[row], tl[tok], bound_k)) {
-            out32[(uint64_t)tok * M + row] = (float)v;
-          } else {  // open: pf_hc_up_fix writes it
-            const uint32_t at = atomicAdd(cnt, 1u);
-            open[2 * at] = tok, open[2 * at + 1] = row;
-          }
-        } else {
-          part[((uint64_t)split * N + tok) * M + row] = v;
-        }
+        int s[kDiagonals];
+#pragma unroll
+        for (uint32_t d = 0; d < kDiagonals; d++) s[d] = acc[i][j][d][q];
+        v[q] = ldexp(diagonals(s), rs[q].exp + ts.exp - 312);
       }
+      if constexpr (kUp) {
+        *(float4 *)(out32 + (uint64_t)tok * M + row) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (!certain(v[q], rs[q], ts, bound_k)) {  // open: pf_hc_up_fix writes it
+            const uint32_t at = atomicAdd(cnt, 1u);
+            open[2 * at] = tok, open[2 * at + 1] = row + q;
+          }
+      } else {
+        double *o = part + ((uint64_t)split * N + tok) * M + row;
+        *(double2 *)o = make_double2(v[0], v[1]), *(double2 *)(o + 2) = make_double2(v[2], v[3]);
+      }
+    }
+  }
 }
 
 // Token t's down sums (rows < lr of W_down, then the 4 of W_inject): the splits added in order, certified against the
@@ -214,13 +322,14 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_gemm(const uint16_t *A0, uint32_t
 // raw entry is written by pf_hc_down_fix). force_open sends all.
 __global__ void __launch_bounds__(kHcWG) pf_hc_down_fin(const double *part, uint32_t T, uint32_t M, uint32_t nsplit,
                                                         const double *rn, const double *tn, const int *rl,
-                                                        const int *tl, double bound_k, bool force_open, float *raw,
-                                                        uint32_t *open, uint32_t *cnt) {
+                                                        const int *tl, HcGrid gr, HcGrid gt, double bound_k,
+                                                        bool force_open, float *raw, uint32_t *open, uint32_t *cnt) {
   const uint32_t t = blockIdx.x;
+  const Side ts = side_of(tn, tl, gt, t);
   for (uint32_t row = threadIdx.x; row < M; row += kHcWG) {
     double v = 0.0;
     for (uint32_t s = 0; s < nsplit; s++) v = __dadd_rn(v, part[((uint64_t)s * T + t) * M + row]);
-    if (!force_open && certain(v, rn[row], tn[t], rl[row], tl[t], bound_k)) {
+    if (!force_open && certain(v, side_of(rn, rl, gr, row), ts, bound_k)) {
       raw[(uint64_t)t * M + row] = (float)v;
     } else {
       const uint32_t at = atomicAdd(cnt, 1u);
@@ -302,13 +411,13 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_up_fix(const uint16_t *w_up, uint
 }
 
 // Token t: l = silu(v / 4) for W_down's rows (the quarter exact; z / (1 + e^-z)) as bf16 bits (the up GEMM's operand),
-// the inject logits for W_inject's, and the 2-norm (rounded up) and least lsb exponent of bf16(l).
+// the inject logits for W_inject's, and the 2-norm (rounded up), least lsb exponent and largest exponent field of bf16(l).
 __global__ void __launch_bounds__(kHcWG) pf_hc_down_epi(const float *raw, uint32_t lr, uint16_t *lb, float *inj,
-                                                        double *ln, int *llsb) {
+                                                        double *ln, int *llsb, HcGrid l) {
   __shared__ uint64_t tab[32];
   __shared__ double red[4];
   __shared__ int redi[4];
-  int lsb = 1 << 20;
+  int lsb = 1 << 20, top = 0;
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
   __syncthreads();
   const uint32_t t = blockIdx.x, M = lr + kHcStreams4;
@@ -323,12 +432,15 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_down_epi(const float *raw, uint32
       const double b = (double)bo;
       sq = __builtin_fma(b, b, sq);
       lsb = min(lsb, bf16_lsb_of(bo));
+      top = max(top, (int)((__float_as_uint(bo) >> 23) & 0xffu));
     } else {
       inj[(uint64_t)t * kHcStreams4 + j - lr] = v;
     }
   }
   sq = wg_sum(sq, red);
   lsb = wg_min(lsb, redi);
+  top = -wg_min(-top, redi);
+  if (threadIdx.x == 0) l.exp[t] = top;
   if (threadIdx.x == 0) ln[t] = sqrt(sq) * (1.0 + 0x1p-30), llsb[t] = lsb;
 }
 
@@ -393,27 +505,37 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_post(float *R, const float *y, co
 hipError_t prefill_hc_pre(const HcShape &S, const HcLayer &L, const HcBufs &b, const float *R, bool force_open,
                           hipStream_t st) {
   const uint32_t H = S.H, lr = S.lr, T = S.T, D = kHcStreams4 * H, Md = lr + kHcStreams4;
-  pf_hc_norm<<<T, kHcWG, 0, st>>>(R, L.gamma, H, b.sc, b.nb, b.nn, b.nlsb, b.cnt);
-  // The down GEMM: K = 4H in kHcDownSplit parts. Roundings on a sum's path: here at most 4 per matrix-core step over a
-  // kGroupK chain, one per group total, one per split; in the fixed order 8 (chain) + 1 + 3 (tree) + K / 2048 (the
-  // slot's chunks) + 16 (the slots); doubled, and 2^-53 each.
-  const uint32_t ksplit = (D / kHcDownSplit + kGroupK - 1) / kGroupK * kGroupK;
-  const double nd = 2.0 * (4.0 * (kGroupK / 4) + D / kGroupK + kHcDownSplit + 28.0 + D / 2048.0);
-  const dim3 gd(((Md + 63) / 64) * ((T + 63) / 64), kHcDownSplit);
-  pf_hc_gemm<false><<<gd, kHcWG, 0, st>>>(L.w_down, lr, L.w_inj, Md, D, b.nb, T, ksplit, b.part, nullptr, nullptr,
-                                          nullptr, nullptr, nullptr, 0.0, nullptr, nullptr);
-  pf_hc_down_fin<<<T, kHcWG, 0, st>>>(b.part, T, Md, kHcDownSplit, L.row_norm, b.nn, L.row_lsb, b.nlsb,
-                                      nd * 0x1p-53, force_open, b.raw, b.open, b.cnt);
+  const uint32_t nd = D / 64, nu = (lr + 63) / 64, tiles = (T + 15) / 16;
+  pf_hc_norm<<<T, kHcWG, 0, st>>>(R, L.gamma, H, b.sc, b.nb, b.nn, b.nlsb, b.ng, b.lg, b.cnt);
+  pf_hc_digits<<<dim3(tiles, (nd + 3) / 4), kHcWG, 0, st>>>(b.nb, T, nullptr, T, D, b.ng, b.nd);
+  // The down GEMM: K = 4H in kHcDownSplit parts. Roundings on a sum's path: here one a part and one a part's addition; in
+  // the fixed order 8 (chain) + 1 + 3 (tree) + K / 2048 (the slot's chunks) + 16 (the slots); doubled, and 2^-53 each.
+  const double bd = 2.0 * (1.0 + kHcDownSplit + 28.0 + D / 2048.0);
+  pf_hc_gemm<false><<<(Md + 63) / 64 * ((T + 63) / 64) * kHcDownSplit, kHcWG, 0, st>>>(
+      L.dig_down, Md, b.nd, T, nd, kHcDownSplit, b.part, nullptr, nullptr, nullptr, nullptr, nullptr, L.grid, b.ng, 0.0, nullptr,
+      nullptr);
+  pf_hc_down_fin<<<T, kHcWG, 0, st>>>(b.part, T, Md, kHcDownSplit, L.row_norm, b.nn, L.row_lsb, b.nlsb, L.grid, b.ng,
+                                      bd * 0x1p-53, force_open, b.raw, b.open, b.cnt);
   pf_hc_down_fix<<<256, kHcWG, 0, st>>>(L.w_down, L.w_inj, lr, D, b.nb, b.open, b.cnt, b.raw);
-  pf_hc_down_epi<<<T, kHcWG, 0, st>>>(b.raw, lr, b.lb, b.inj, b.ln, b.llsb);
+  pf_hc_down_epi<<<T, kHcWG, 0, st>>>(b.raw, lr, b.lb, b.inj, b.ln, b.llsb, b.lg);
   // The up GEMM: 4H rows of W_up against bf16(l), K = lr; the fixed order is a k chain of lr terms.
-  const double nu = 2.0 * (4.0 * (kGroupK / 4) + lr / (double)kGroupK + 1.0 + lr);
-  const dim3 gu(((D + 63) / 64) * ((T + 63) / 64), 1);
-  pf_hc_gemm<true><<<gu, kHcWG, 0, st>>>(L.w_up, D, nullptr, D, lr, b.lb, T, lr, nullptr, b.a, L.row_norm + Md, b.ln,
-                                         L.row_lsb + Md, b.llsb, nu * 0x1p-53, b.open_up, b.cnt + 1);
+  pf_hc_digits<<<dim3(tiles, (nu + 3) / 4), kHcWG, 0, st>>>(b.lb, T, nullptr, T, lr, b.lg, b.ld);
+  const double bu = 2.0 * (1.0 + 1.0 + lr);
+  const HcGrid gu{L.grid.exp + Md, L.grid.lost + Md};
+  pf_hc_gemm<true><<<(D + 63) / 64 * ((T + 63) / 64), kHcWG, 0, st>>>(L.dig_up, D, b.ld, T, nu, 1, nullptr, b.a,
+                                                                      L.row_norm + Md, b.ln, L.row_lsb + Md, b.llsb, gu, b.lg,
+                                                                      bu * 0x1p-53, b.open_up, b.cnt + 1);
   pf_hc_up_fix<<<256, kHcWG, 0, st>>>(L.w_up, lr, D, b.lb, b.open_up, b.cnt + 1, b.a);
   const uint64_t nx = (uint64_t)T * H;
   pf_hc_mix<<<(uint32_t)((nx + 2 * kHcWG - 1) / (2 * kHcWG)), kHcWG, 0, st>>>(R, L.gamma, b.sc, b.a, T, H, b.x);
+  return hipGetLastError();
+}
+
+hipError_t prefill_hc_load(uint32_t H, uint32_t lr, const HcLayer &L, uint8_t *dig_down, uint8_t *dig_up, hipStream_t st) {
+  const uint32_t D = kHcStreams4 * H, Md = lr + kHcStreams4;
+  pf_hc_digits<<<dim3((Md + 15) / 16, (D / 64 + 3) / 4), kHcWG, 0, st>>>(L.w_down, lr, L.w_inj, Md, D, L.grid, dig_down);
+  pf_hc_digits<<<dim3(D / 16, ((lr + 63) / 64 + 3) / 4), kHcWG, 0, st>>>(L.w_up, D, nullptr, D, lr,
+                                                                         HcGrid{L.grid.exp + Md, L.grid.lost + Md}, dig_up);
   return hipGetLastError();
 }
 

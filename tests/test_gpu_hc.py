@@ -61,7 +61,7 @@ def test_forward_hc_requires_module():
 @pytest.mark.parametrize("shape", [(512, 256, 32, 4, 64), (2560, 640, 64, 8, 320)])
 @pytest.mark.parametrize("fixed_order", [False, True])
 def test_forward_hc_prefill(shape, fixed_order):
-    """More tokens than the decode kernel takes: the mix's kernels (fp64 matrix cores within a bound, the open sums in
+    """More tokens than the decode kernel takes: the mix's kernels (exact digit products within a bound, the open sums in
     the fixed order; with hc_fixed_order every down sum in the fixed order), the prefill block, the combine's kernel;
     R, y and the routing against the oracle's, bit for bit (the exact router: the oracle's weights and y)."""
     H, F, E, K, lr = shape
@@ -83,3 +83,43 @@ def test_forward_hc_prefill(shape, fixed_order):
         assert np.array_equal(y, yo), (T, h.max_abs(y, yo))
         assert np.array_equal(R2, Ro), (T, h.max_abs(R2, Ro))
     blk.close()
+
+
+@pytest.mark.parametrize("lr,T", [(8, 17), (72, 63), (328, 65), (512, 49)])
+def test_forward_hc_prefill_wide_values(lr, T):
+    """The mix's digit products at their edges: ranks and tokens that end inside a 64-value chunk, a 16-row tile and a 64-row
+    tile; rows and tokens whose values span 2^50 (they lose bits of their grid), whose largest value is a power of two or a
+    subnormal, all-zero rows and tokens; R, y and the routing against the oracle's, bit for bit."""
+    H, F, E, K = 512, 256, 32, 4
+    say("forward_hc prefill wide values, rank", lr, "T", T)
+    L = h.Layer(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, moe.QT_Q8_0, moe.QT_Q8_0, seed=lr, zipf=1.1)
+    hc = h.HcModule(H, lr, seed=13)
+    r = np.random.default_rng(lr + T)
+
+    def widen(w):
+        f = (w.astype(np.uint32) << 16).view(np.float32).copy()
+        f[::3] *= np.exp2(-r.integers(0, 50, f[::3].shape)).astype(np.float32)  # spans 2^50
+        f[1::7] = 0.0
+        f[2::7] = np.where(r.random(f[2::7].shape) < 0.5, np.float32(-0.25), np.float32(2.0 ** -24))
+        f[4::11, 0] = 2.0 ** -130
+        f[5::11] *= np.float32(2.0 ** -120)
+        return h.to_bf16(f.reshape(-1)).reshape(w.shape)
+
+    hc.down, hc.inj, hc.up = widen(hc.down), widen(hc.inj), widen(hc.up)
+    blk = moe.MoeBlock(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, True, moe.QT_Q8_0, moe.QT_Q8_0, n_layer=1, max_tokens=T,
+                       hc_lr=lr, exact_router=True)
+    L.upload(blk, 0)
+    hc.load(blk, 0)
+    R = r.standard_normal((T, 4, H)).astype(np.float32)
+    R[::4] *= np.exp2(-r.integers(0, 50, R[::4].shape)).astype(np.float32)
+    R[3] = 0.0
+    R[5] = np.where(r.random((4, H)) < 0.5, np.float32(1.0), np.float32(-1.0))
+    R[6, :, 1:] = 0.0
+    R2, y, ids, w = blk.forward_hc(0, R)
+    x, inj = hc.pre(R)
+    yo, io, wo = L.oracle_forward(x)
+    Ro = h.HcModule.post(R, inj, yo)
+    blk.close()
+    assert np.array_equal(ids, io) and np.array_equal(w, wo)
+    assert np.array_equal(y, yo), h.max_abs(y, yo)
+    assert np.array_equal(R2, Ro), h.max_abs(R2, Ro)
