@@ -12,7 +12,7 @@
 // it is the fixed order's rounding; and where the products' bits span fewer than 53 (the least lsb of the row's and of
 // the token's values against the Cauchy-Schwarz bound on sum|p|), both sums are exact, whatever their order (ties of
 // fp32 rounding are common for W_up's short sums, and this settles them).
-// Otherwise the sum is recomputed in the fixed order, one wave an open sum, from a list, in a kernel of its own:
+// Otherwise the sum is recomputed in the fixed order, from a list, in a kernel of its own:
 // W_up's a k-order chain of at most 512 terms, W_down's and W_inject's the decode kernel's 512-value-chunk tree.
 #include <hip/hip_runtime.h>
 
@@ -63,45 +63,61 @@ __device__ __forceinline__ int wg_min(int v, int *red) {
   return m;
 }
 
-// Token t (one work-group): each stream as RMSNorm(R_s) gamma_s, the decode kernel's hc_norm_item arithmetic (each
-// thread's squares in order, then wg_sum; mean rounded to fp32; 1 / sqrtf(mean + 1e-6)): the stream's scale into sc
+// Token t (one work-group, 256 threads a stream): each stream as RMSNorm(R_s) gamma_s, the decode kernel's hc_norm_item
+// arithmetic (each thread's squares in order, then the stream's sum in wg_sum's order; mean rounded to fp32;
+// 1 / sqrtf(mean + 1e-6)): the stream's scale into sc
 // (pf_hc_mix forms n again from R, the scale and gamma), bf16(n) into nb, and the 2-norm (rounded up), least lsb
 // exponent and largest exponent field of bf16(n). Work-group 0 clears the open lists' counts, each its token's counts of
-// values that lose bits.
-__global__ void __launch_bounds__(kHcWG) pf_hc_norm(const float *R, const float *gamma, uint32_t H, float *sc,
-                                                    uint16_t *nb, double *nn, int *nlsb, HcGrid n, HcGrid l,
-                                                    uint32_t *cnt) {
-  __shared__ double red[4];
-  __shared__ int redi[4];
-  int lsb = 1 << 20, top = 0;
-  const uint32_t t = blockIdx.x;
+// values that lose bits. Latency bound (a thread's H / 256 loads, the sum's exchanges): the four streams side by side
+// instead of one after another take 23 us at 1000 tokens of H 2560, 39 before.
+__global__ void __launch_bounds__(kHcStreams4 * kHcWG) pf_hc_norm(const float *R, const float *gamma, uint32_t H, float *sc,
+                                                                  uint16_t *nb, double *nn, int *nlsb, HcGrid n, HcGrid l,
+                                                                  uint32_t *cnt) {
+  __shared__ double red[kHcStreams4][4];
+  __shared__ int redi[2][kHcStreams4 * 4];
+  const uint32_t t = blockIdx.x, s = threadIdx.x / kHcWG, i0 = threadIdx.x % kHcWG, wv = threadIdx.x >> 6;
   if (t == 0 && threadIdx.x < 2) cnt[threadIdx.x] = 0u;
   if (threadIdx.x == 0) n.lost[t] = l.lost[t] = 0u;
+  // v summed over the stream's 256 threads, as wg_sum.
+  const auto stream_sum = [&](double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = __dadd_rn(v, __shfl_xor(v, o, 64));
+    __syncthreads();
+    if (lane_of() == 0) red[s][wv % 4] = v;
+    __syncthreads();
+    return __dadd_rn(__dadd_rn(red[s][0], red[s][1]), __dadd_rn(red[s][2], red[s][3]));
+  };
+  const float *r = R + ((uint64_t)t * kHcStreams4 + s) * H;
+  double ss = 0.0;
+#pragma unroll 2
+  for (uint32_t i = i0; i < H; i += kHcWG) ss = __dadd_rn(ss, (double)__fmul_rn(r[i], r[i]));
+  ss = stream_sum(ss);
+  const float mean = (float)(ss / (double)H);
+  const float scale = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, 1e-6f)));
+  if (i0 == 0) sc[t * kHcStreams4 + s] = scale;
+  uint16_t *ob = nb + ((uint64_t)t * kHcStreams4 + s) * H;
   double sq = 0.0;
-  for (uint32_t s = 0; s < kHcStreams4; s++) {
-    const float *r = R + ((uint64_t)t * kHcStreams4 + s) * H;
-    double ss = 0.0;
-    for (uint32_t i = threadIdx.x; i < H; i += kHcWG) ss = __dadd_rn(ss, (double)__fmul_rn(r[i], r[i]));
-    ss = wg_sum(ss, red);
-    const float mean = (float)(ss / (double)H);
-    const float scale = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, 1e-6f)));
-    if (threadIdx.x == 0) sc[t * kHcStreams4 + s] = scale;
-    uint16_t *ob = nb + ((uint64_t)t * kHcStreams4 + s) * H;
-    for (uint32_t i = threadIdx.x; i < H; i += kHcWG) {
-      const float v = __fmul_rn(__fmul_rn(r[i], scale), gamma[s * H + i]);
-      const float bv = round_bf16(v);
-      ob[i] = (uint16_t)(__float_as_uint(bv) >> 16);
-      const double b = (double)bv;
-      sq = __builtin_fma(b, b, sq);
-      lsb = min(lsb, bf16_lsb_of(bv));
-      top = max(top, (int)((__float_as_uint(bv) >> 23) & 0xffu));
-    }
+  int lsb = 1 << 20, top = 0;
+#pragma unroll 2
+  for (uint32_t i = i0; i < H; i += kHcWG) {
+    const float v = __fmul_rn(__fmul_rn(r[i], scale), gamma[s * H + i]);
+    const float bv = round_bf16(v);
+    ob[i] = (uint16_t)(__float_as_uint(bv) >> 16);
+    const double b = (double)bv;
+    sq = __builtin_fma(b, b, sq);
+    lsb = min(lsb, bf16_lsb_of(bv));
+    top = max(top, (int)((__float_as_uint(bv) >> 23) & 0xffu));
   }
-  sq = wg_sum(sq, red);
-  lsb = wg_min(lsb, redi);
-  top = -wg_min(-top, redi);
-  if (threadIdx.x == 0) n.exp[t] = top;
-  if (threadIdx.x == 0) nn[t] = sqrt(sq) * (1.0 + 0x1p-30), nlsb[t] = lsb;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) lsb = min(lsb, __shfl_xor(lsb, o, 64)), top = max(top, __shfl_xor(top, o, 64));
+  if (lane_of() == 0) redi[0][wv] = lsb, redi[1][wv] = top;
+  (void)stream_sum(sq);
+  if (threadIdx.x == 0) {
+    double q = 0.0;
+    for (uint32_t k = 0; k < kHcStreams4; k++) q = __dadd_rn(q, __dadd_rn(__dadd_rn(red[k][0], red[k][1]), __dadd_rn(red[k][2], red[k][3])));
+    for (uint32_t k = 0; k < kHcStreams4 * 4; k++) lsb = min(lsb, redi[0][k]), top = max(top, redi[1][k]);
+    nn[t] = sqrt(q) * (1.0 + 0x1p-30), nlsb[t] = lsb, n.exp[t] = top;
+  }
 }
 
 // Four values' digits (X as bytes after the carry trick below) as four words of one digit each.
@@ -184,13 +200,12 @@ __device__ __forceinline__ bool certain(double v, const Side &r, const Side &t, 
   return (float)(v - bnd) == f && (float)(v + bnd) == f;
 }
 
-// sum of s[i] 256^i, rounded to fp64 once: the low three and the high four weights as 64-bit integers, then 2^40 h + l
-// with both parts exact in fp64.
+// sum of s[i] 256^i, rounded to fp64 once: a part has at most 4096 values, so |s[6]| <= 2^24, |s[5]| <= 2^26, |s[4]| <= 2^27,
+// |s[3]| and |s[2]| < 2^28, |s[1]| <= 2^27, |s[0]| <= 2^26, and every step but the last is exact.
 __device__ __forceinline__ double diagonals(const int s[kDiagonals]) {
-  const int64_t lo = (int64_t)s[0] + ((int64_t)s[1] << 8) + ((int64_t)s[2] << 16);
-  const int64_t hi = (int64_t)s[3] + ((int64_t)s[4] << 8) + ((int64_t)s[5] << 16) + ((int64_t)s[6] << 24) + (lo >> 24);
-  const uint64_t l40 = ((uint64_t)(hi & 0xffff) << 24) | (uint64_t)(lo & 0xffffff);
-  return __builtin_fma((double)(hi >> 16), 0x1p40, (double)l40);
+  const double p = __builtin_fma((double)s[6], 256.0, (double)s[5]), q = __builtin_fma((double)s[4], 256.0, (double)s[3]);
+  const double r = __builtin_fma((double)s[2], 65536.0, __builtin_fma((double)s[1], 256.0, (double)s[0]));
+  return __builtin_fma(__builtin_fma(p, 65536.0, q), 0x1p24, r);
 }
 
 // C = A B^T over the digits of the rows (M of them, A) and of the tokens (N, B), nch 64-value chunks in blockIdx.x % nsplit
@@ -203,7 +218,7 @@ __device__ __forceinline__ double diagonals(const int s[kDiagonals]) {
 // takes every eighth row tile.
 // kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
 // (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M).
-// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 52 us and up 65, where the fp64 matrix cores took 162 and 141.
+// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 51 us and up 59, where the fp64 matrix cores took 162 and 141.
 template <bool kUp>
 __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
                                                        uint32_t nch, uint32_t nsplit, double *part, float *out32,
@@ -341,17 +356,19 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_down_fin(const double *part, uint
 // The open down sums in the decode kernel's fixed order (bf16_dot for one row and one token, restated for one wave):
 // 512-value chunks c; lane l's eight values 8 l .. 8 l + 7 a fused chain from zero; a lane row r (16 lanes) as
 // ((P0 + P7) + (P3 + P4)) + ((P1 + P6) + (P2 + P5)), P_m = a_m + a_(15 - m); slot 4 (c mod 4) + r takes the chunks'
-// sums in chunk order; the 16 slots added in order from zero. One wave an entry.
+// sums in chunk order; the 16 slots added in order from zero. A work-group an entry, wave q the chunks q, q + 4, ..: what
+// bounds it is one entry's chunk chain (K = 10240, 1000 tokens: 9.5 us, one wave an entry 24).
 __global__ void __launch_bounds__(kHcWG) pf_hc_down_fix(const uint16_t *w_down, const uint16_t *w_inj, uint32_t lr,
                                                         uint32_t K, const uint16_t *nb, const uint32_t *open,
                                                         const uint32_t *cnt, float *raw) {
-  const uint32_t lane = lane_of(), r = lane / 16, nw = gridDim.x * (kHcWG / 64), M = lr + kHcStreams4;
-  for (uint32_t e = blockIdx.x * (kHcWG / 64) + (threadIdx.x >> 6); e < *cnt; e += nw) {
+  __shared__ double slots[16];  // slot 4 q + r
+  const uint32_t lane = lane_of(), r = lane / 16, q = threadIdx.x >> 6, M = lr + kHcStreams4;
+  for (uint32_t e = blockIdx.x; e < *cnt; e += gridDim.x) {
     const uint32_t t = open[2 * e], row = open[2 * e + 1];
     const uint16_t *wr = row < lr ? w_down + (uint64_t)row * K : w_inj + (uint64_t)(row - lr) * K;
     const uint16_t *xr = nb + (uint64_t)t * K;
-    double slot[4] = {0.0, 0.0, 0.0, 0.0};  // slot 4 w + r, w = c mod 4 (lane 16 r holds its row's)
-    for (uint32_t c = 0; c < K / 512; c++) {
+    double slot = 0.0;
+    for (uint32_t c = q; c < K / 512; c += 4) {
       const uint32_t k0 = 512 * c + 8 * lane;
       const uint4 wq = *(const uint4 *)(wr + k0), xq = *(const uint4 *)(xr + k0);
       const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w}, xw[4] = {xq.x, xq.y, xq.z, xq.w};
@@ -365,16 +382,16 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_down_fix(const uint16_t *w_down, 
       for (int j = 0; j < 8; j++) p[j] = __shfl(P, (int)(16 * r + j), 64);
       const double S = __dadd_rn(__dadd_rn(__dadd_rn(p[0], p[7]), __dadd_rn(p[3], p[4])),
                                  __dadd_rn(__dadd_rn(p[1], p[6]), __dadd_rn(p[2], p[5])));
-#pragma unroll
-      for (uint32_t q = 0; q < 4; q++)
-        if ((c & 3u) == q) slot[q] = c < 4 ? S : __dadd_rn(slot[q], S);
+      slot = c < 4 ? S : __dadd_rn(slot, S);
     }
-    double s = 0.0;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; q++)
-#pragma unroll
-      for (uint32_t rr = 0; rr < 4; rr++) s = __dadd_rn(s, __shfl(slot[q], (int)(16 * rr), 64));
-    if (lane == 0) raw[(uint64_t)t * M + row] = (float)s;
+    if (lane % 16 == 0) slots[4 * q + r] = slot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double s = 0.0;
+      for (uint32_t i = 0; i < 16; i++) s = __dadd_rn(s, slots[i]);
+      raw[(uint64_t)t * M + row] = (float)s;
+    }
+    __syncthreads();
   }
 }
 
@@ -506,7 +523,7 @@ hipError_t prefill_hc_pre(const HcShape &S, const HcLayer &L, const HcBufs &b, c
                           hipStream_t st) {
   const uint32_t H = S.H, lr = S.lr, T = S.T, D = kHcStreams4 * H, Md = lr + kHcStreams4;
   const uint32_t nd = D / 64, nu = (lr + 63) / 64, tiles = (T + 15) / 16;
-  pf_hc_norm<<<T, kHcWG, 0, st>>>(R, L.gamma, H, b.sc, b.nb, b.nn, b.nlsb, b.ng, b.lg, b.cnt);
+  pf_hc_norm<<<T, kHcStreams4 * kHcWG, 0, st>>>(R, L.gamma, H, b.sc, b.nb, b.nn, b.nlsb, b.ng, b.lg, b.cnt);
   pf_hc_digits<<<dim3(tiles, (nd + 3) / 4), kHcWG, 0, st>>>(b.nb, T, nullptr, T, D, b.ng, b.nd);
   // The down GEMM: K = 4H in kHcDownSplit parts. Roundings on a sum's path: here one a part and one a part's addition; in
   // the fixed order 8 (chain) + 1 + 3 (tree) + K / 2048 (the slot's chunks) + 16 (the slots); doubled, and 2^-53 each.
@@ -516,7 +533,7 @@ hipError_t prefill_hc_pre(const HcShape &S, const HcLayer &L, const HcBufs &b, c
       nullptr);
   pf_hc_down_fin<<<T, kHcWG, 0, st>>>(b.part, T, Md, kHcDownSplit, L.row_norm, b.nn, L.row_lsb, b.nlsb, L.grid, b.ng,
                                       bd * 0x1p-53, force_open, b.raw, b.open, b.cnt);
-  pf_hc_down_fix<<<256, kHcWG, 0, st>>>(L.w_down, L.w_inj, lr, D, b.nb, b.open, b.cnt, b.raw);
+  pf_hc_down_fix<<<1024, kHcWG, 0, st>>>(L.w_down, L.w_inj, lr, D, b.nb, b.open, b.cnt, b.raw);
   pf_hc_down_epi<<<T, kHcWG, 0, st>>>(b.raw, lr, b.lb, b.inj, b.ln, b.llsb, b.lg);
   // The up GEMM: 4H rows of W_up against bf16(l), K = lr; the fixed order is a k chain of lr terms.
   pf_hc_digits<<<dim3(tiles, (nu + 3) / 4), kHcWG, 0, st>>>(b.lb, T, nullptr, T, lr, b.lg, b.ld);
