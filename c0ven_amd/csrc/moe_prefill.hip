@@ -23,7 +23,7 @@
 
 namespace c0ven {
 
-constexpr uint32_t kMaxRouteExperts = 512;  // routed experts a layer may have
+constexpr uint32_t kMaxRouteUsed = 17;  // the ranks a token's selection may need: 16 and the next one
 
 __device__ __constant__ static const uint32_t kIq3sGridPf[512] = {C0VEN_IQ3S_GRID_VALUES};
 
@@ -219,6 +219,7 @@ __global__ void __launch_bounds__(kPfWG) pf_topk(const float *logits, uint32_t T
                                                  int32_t *ids, float *w, float *gs, unsigned long long *masks,
                                                  int32_t *ids_out, float *w_out) {
   __shared__ uint64_t tab[32];
+  __shared__ uint2 sel[kPfWG / 64][64 * kRoutePer + kMaxRouteUsed];
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
   __syncthreads();
   const uint32_t t = blockIdx.x * (kPfWG / 64) + wave_id(), lane = lane_id();
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(kPfWG) pf_topk(const float *logits, uint32_t T
   route_load<false>(lg, E, lane, key, id);
   float mx, inv;
   route_norm(key, E, lane, tab, &mx, &inv);
-  route_select(key, id, K, lane, &my_id, &my_key);
+  route_select_lds(key, id, K, lane, sel[wave_id()], &my_id, &my_key);
   const float wk = route_weight(my_key, mx, inv, K, lane, tab);
   if (lane < K) {
     ids[(uint64_t)t * K + lane] = (int32_t)my_id;
@@ -464,13 +465,13 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
                                                       unsigned long long *masks, uint32_t *cnt_exact,
                                                       int32_t *ids_out, float *w_out) {
   __shared__ uint64_t tab[32];
-  __shared__ uint32_t cand[kPfWG / 64][kMaxRouteExperts];
-  __shared__ uint32_t xkey[kPfWG / 64][kMaxRouteExperts];  // 0, or an exactly summed expert's key (cleared after)
+  // A wave's: route_select_lds's candidates; between its two uses the experts to sum, and for each 0 or its exact key.
+  __shared__ uint2 sel[kPfWG / 64][64 * kRoutePer + kMaxRouteUsed];
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
-  for (uint32_t i = threadIdx.x; i < (kPfWG / 64) * kMaxRouteExperts; i += kPfWG) (&xkey[0][0])[i] = 0u;
   __syncthreads();
   const uint32_t t = blockIdx.x * (kPfWG / 64) + wave_id(), lane = lane_id(), wv = wave_id();
   if (t >= T) return;
+  uint32_t *const cand = (uint32_t *)sel[wv], *const xkey = cand + 64 * kRoutePer;
   float *lg = logits + (uint64_t)t * (E + 1);
   uint32_t key[kRoutePer], id[kRoutePer], my_id, my_key;
   route_load<false>(lg, E, lane, key, id);
@@ -480,14 +481,9 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
   for (int i = 0; i < kRoutePer; i++) mk = max(mk, lane + 64 * i < E ? float_key(fabsf(key_float(key[i]))) : 0u);
   const double labs = (double)key_float(wave_max_u32(mk));
   const double B = (double)gamma_rmax * (double)xn[t] + 0x1p-22 * (labs + (double)bias_max) + 1e-30;
-  // The K + 1 largest (lane r < K + 1: rank r), on a copy of the keys.
+  // The K + 1 largest (lane r < K + 1: rank r).
   const uint32_t K1 = K < E ? K + 1 : K;
-  {
-    uint32_t kc[kRoutePer], ic[kRoutePer];
-#pragma unroll
-    for (int i = 0; i < kRoutePer; i++) kc[i] = key[i], ic[i] = id[i];
-    route_select(kc, ic, K1, lane, &my_id, &my_key);
-  }
+  route_select_lds(key, id, K1, lane, sel[wv], &my_id, &my_key);
   const double v = (double)key_float(my_key);
   const double nxt = __shfl_down(v, 1, 64), prv = __shfl_up(v, 1, 64);
   // Rank r's order against rank r + 1 is open when their intervals (each +- B) meet.
@@ -501,9 +497,11 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
     const double thr = __shfl(v, (int)K - 1, 64) - 2.0 * B;
     const uint32_t kK = __shfl(my_key, (int)K, 64), iK = __shfl(my_id, (int)K, 64);
     uint32_t nc = 0;
+#pragma unroll
+    for (int i = 0; i < kRoutePer; i++) xkey[lane + 64 * i] = 0u;
     {
       const uint64_t bal = __ballot(amb);
-      if (amb) cand[wv][__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = my_id;
+      if (amb) cand[__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = my_id;
       nc = (uint32_t)__popcll(bal);
     }
 #pragma unroll
@@ -512,34 +510,42 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
       const bool after = key[i] < kK || (key[i] == kK && e > iK);  // ranked after the (K + 1)-th
       const bool c = kopen && e < E && after && (double)key_float(key[i]) >= thr;
       const uint64_t bal = __ballot(c);
-      if (c) cand[wv][nc + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = e;
+      if (c) cand[nc + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = e;
       nc += (uint32_t)__popcll(bal);
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
-    // Sixteen lanes a candidate: lane s of group j sums the row's sixteenth s in fp64 (its magnitudes too, and the
-    // least exponent sum of its products), the group adds its sixteen partials in a fixed tree; exact when the
-    // magnitudes' sum is below 2^(lsb + 53). x's bf16 row is read from memory (L2) by each candidate's group: staged
-    // in LDS (32 KB a work-group) it measured ~1 us slower at config 4, and kept the kernel off CUs whose LDS the
-    // shared expert's launches beside it hold.
+    // Sixteen lanes a candidate: lane s of group j sums every sixteenth 16-byte piece of the row from s on in fp64 (its
+    // magnitudes too, in fp32, and the least exponent sum of its products), the group adds its sixteen partials in a
+    // fixed tree; exact when the magnitudes' sum is below 2^(lsb + 53). What bounds the kernel is this path's latency in
+    // the few tokens that take it (2048 tokens of H 2048: 16.4 us, 20.6 with a sixteenth of the row in one lane and
+    // products and magnitudes in fp64, 11 with no token open). x's bf16 row is read from memory (L2) by each
+    // candidate's group: staged in LDS (32 KB a work-group) it measured ~1 us slower, and kept the kernel off CUs whose
+    // LDS the shared expert's launches beside it hold.
     const uint4 *xs = (const uint4 *)(xb + (uint64_t)t * H);
-    const uint32_t j = lane / 16, sl = lane % 16, H16 = H / 16;  // H16 / 8 pieces of 16 B a lane
+    const uint32_t j = lane / 16, sl = lane % 16, np = H / 128;  // a lane's 16-byte pieces: sl, sl + 16, ..
     for (uint32_t c0 = 0; c0 < nc; c0 += 4) {
-      const uint32_t ci = c0 + j, e = cand[wv][min(ci, nc - 1)];
-      const uint4 *wr = (const uint4 *)(W + (uint64_t)e * H + sl * H16);
-      const uint4 *xr = xs + sl * H16 / 8;
+      const uint32_t ci = c0 + j, e = cand[min(ci, nc - 1)];
+      const uint4 *wr = (const uint4 *)(W + (uint64_t)e * H) + sl;
+      const uint4 *xr = xs + sl;
       // Four chains (piece q % 4): when the sum is exact (checked below) every order gives it, so the chains and the
       // tree that joins them need not follow k.
-      double acc4[4] = {0.0, 0.0, 0.0, 0.0}, mag4[4] = {0.0, 0.0, 0.0, 0.0};
+      // A product is formed in fp32, exact when no bit of it lies below 2^-149 (checked with the rest), and its magnitude
+      // summed there: a few hundred roundings, covered by the test's factor.
+      double acc4[4] = {0.0, 0.0, 0.0, 0.0};
+      float mag4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       uint32_t emin = 0xffffffffu;  // the least sum of the two exponent fields of a product, two 16-bit halves
-      for (uint32_t k0 = 0; k0 < H16 / 8; k0 += 16) {  // sixteen pieces of the row in flight at a time
-        uint4 a[16];
+      for (uint32_t k0 = 0; k0 < np; k0 += 8) {  // eight pieces of the row and of x in flight at a time
+        uint4 a[8], b[8];
 #pragma unroll
-        for (int q = 0; q < 16; q++) a[q] = k0 + q < H16 / 8 ? wr[k0 + q] : make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t q = 0; q < 8; q++) {
+          const uint32_t k = 16 * min(k0 + q, np - 1);
+          a[q] = wr[k], b[q] = xr[k];
+        }
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-          if (k0 + q >= H16 / 8) break;
-          const uint4 bq = xr[k0 + q];
+        for (uint32_t q = 0; q < 8; q++) {
+          if (k0 + q >= np) continue;
+          const uint4 bq = b[q];
           const uint32_t aw[4] = {a[q].x, a[q].y, a[q].z, a[q].w}, bw[4] = {bq.x, bq.y, bq.z, bq.w};
 #pragma unroll
           for (int i = 0; i < 4; i++) {
@@ -548,42 +554,39 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
             const uint32_t es = ((aw[i] >> 7) & 0x00ff00ffu) + ((bw[i] >> 7) & 0x00ff00ffu);
             emin = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, emin),
                                                                           __builtin_bit_cast(u16x2_t, es)));
-            const double p0 = (double)__uint_as_float(aw[i] << 16) * (double)__uint_as_float(bw[i] << 16);
-            const double p1 = (double)__uint_as_float(aw[i] & 0xffff0000u) * (double)__uint_as_float(bw[i] & 0xffff0000u);
-            acc4[q % 4] = __dadd_rn(__dadd_rn(acc4[q % 4], p0), p1);
-            mag4[q % 4] = __dadd_rn(__dadd_rn(mag4[q % 4], fabs(p0)), fabs(p1));
+            const float p0 = __fmul_rn(__uint_as_float(aw[i] << 16), __uint_as_float(bw[i] << 16));
+            const float p1 = __fmul_rn(__uint_as_float(aw[i] & 0xffff0000u), __uint_as_float(bw[i] & 0xffff0000u));
+            acc4[q % 4] = __dadd_rn(__dadd_rn(acc4[q % 4], (double)p0), (double)p1);
+            mag4[q % 4] = __fadd_rn(__fadd_rn(mag4[q % 4], fabsf(p0)), fabsf(p1));
           }
         }
       }
       double acc = __dadd_rn(__dadd_rn(acc4[0], acc4[1]), __dadd_rn(acc4[2], acc4[3]));
-      double mag = __dadd_rn(__dadd_rn(mag4[0], mag4[1]), __dadd_rn(mag4[2], mag4[3]));
+      float mag = __fadd_rn(__fadd_rn(mag4[0], mag4[1]), __fadd_rn(mag4[2], mag4[3]));
       uint32_t em = min(emin & 0xffffu, emin >> 16);
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) {
         acc = __dadd_rn(acc, __shfl_xor(acc, o, 64));
-        mag = __dadd_rn(mag, __shfl_xor(mag, o, 64));
+        mag = __fadd_rn(mag, __shfl_xor(mag, o, 64));
         em = min(em, (uint32_t)__shfl_xor((int)em, o, 64));
       }
       // Every product is a multiple of 2^(em - 268) (exponent fields less 127 each, less 7 mantissa bits each), and of
       // 2^(rlsb + xlsb): exact when the magnitudes' sum stays below 2^53 times the larger of the two.
       const int lsb = max((int)em - 268, rlsb[e] + xlsb[t]);
-      const bool exact_ok = mag * (1.0 + 0x1p-40) < ldexp(1.0, lsb + 53);
+      const bool exact_ok = lsb >= -149 && (double)mag * (1.0 + 0x1p-10) < ldexp(1.0, lsb + 53);
       float lgv = (float)acc;
       if (!exact_ok && sl == 0 && ci < nc) lgv = exact_logit_chain(W, xb, H, e, t);
-      if (sl == 0 && ci < nc) xkey[wv][e] = float_key(bias ? __fadd_rn(lgv, bias[e]) : lgv);
+      if (sl == 0 && ci < nc) xkey[e] = float_key(bias ? __fadd_rn(lgv, bias[e]) : lgv);
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < kRoutePer; i++) {
       const uint32_t e = lane + 64 * i;
-      if (e < E && xkey[wv][e] != 0u) key[i] = xkey[wv][e], xkey[wv][e] = 0u;
+      if (e < E && xkey[e] != 0u) key[i] = xkey[e];
     }
     if (lane == 0) atomicAdd(cnt_exact, 1u);
-    uint32_t kc[kRoutePer], ic[kRoutePer];
-#pragma unroll
-    for (int i = 0; i < kRoutePer; i++) kc[i] = key[i], ic[i] = id[i];
-    route_select(kc, ic, K, lane, &my_id, &my_key);
+    route_select_lds(key, id, K, lane, sel[wv], &my_id, &my_key);
   }
   float mx, inv;
   route_norm(key, E, lane, tab, &mx, &inv);

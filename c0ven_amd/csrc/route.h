@@ -67,41 +67,8 @@ __device__ __forceinline__ double route_sum_part(const uint32_t key[kRoutePer], 
   return wave_sum_f64(acc);
 }
 
-// The top K: lane r < K receives the r-th winner's id and key. Sorts each lane's keys, largest first (ids ascending
-// within a lane, so equal keys keep the lower id first); each round takes the wave's largest head (a DPP max, a
-// ballot for equal keys, the lower id among them) and pops it. key and id are consumed.
-__device__ __forceinline__ void route_select(uint32_t key[kRoutePer], uint32_t id[kRoutePer], uint32_t K,
-                                             uint32_t lane, uint32_t *my_id, uint32_t *my_key) {
-  auto cswap = [&](int i, int j) {
-    const bool sw = (key[j] > key[i]) | ((key[j] == key[i]) & (id[j] < id[i]));  // no short circuit: no branches
-    const uint32_t ki = key[i], ii = id[i];
-    key[i] = sw ? key[j] : ki, id[i] = sw ? id[j] : ii;
-    key[j] = sw ? ki : key[j], id[j] = sw ? ii : id[j];
-  };
-  cswap(0, 1), cswap(2, 3), cswap(4, 5), cswap(6, 7), cswap(0, 2), cswap(1, 3), cswap(4, 6), cswap(5, 7);
-  cswap(1, 2), cswap(5, 6), cswap(0, 4), cswap(3, 7), cswap(1, 5), cswap(2, 6), cswap(1, 4), cswap(3, 6);
-  cswap(2, 4), cswap(3, 5), cswap(3, 4);
-  uint32_t mi = 0, mk = 0;
-  for (uint32_t r = 0; r < K; r++) {
-    const uint32_t m = wave_max_u32(key[0]);
-    const uint64_t cand = __ballot(key[0] == m);
-    uint32_t wid;
-    if (__popcll(cand) == 1) {
-      wid = readlane_u32(id[0], __ffsll((long long)cand) - 1);
-    } else {
-      wid = wave_min_u32(key[0] == m ? id[0] : 0xffffffffu);
-    }
-    if (lane == r) mi = wid, mk = m;
-    if (key[0] == m && id[0] == wid) {  // pop the winner
-#pragma unroll
-      for (int i = 0; i < kRoutePer - 1; i++) key[i] = key[i + 1], id[i] = id[i + 1];
-      key[kRoutePer - 1] = 0;
-    }
-  }
-  *my_id = mi, *my_key = mk;
-}
-
-// The top K as route_select gives them (same winners, same order), by a threshold instead of K rounds: tau, the K-th
+// The top K, largest first, the lower id first among equal keys: lane r < K receives the r-th winner's id and key. By a
+// threshold instead of K rounds of the wave's largest: tau, the K-th
 // largest of the lanes' maxima, is found bit by bit with ballots; at least K keys are >= tau (one a lane of those K
 // lanes), so every winner is among the keys >= tau. Those candidates (usually little more than K) are packed into
 // cand (LDS, room for 64 kRoutePer + K entries) and each is ranked against all of them: rank = the number that beat it
