@@ -131,7 +131,8 @@ __device__ __forceinline__ void transpose4(const uint32_t y[4], uint32_t d[kHcDi
 // The digits of bf16 rows (A0's first M0, then A1's; K values each, a multiple of 8) whose largest exponent fields are
 // g.exp: value (-1)^s m 2^(e - 134) is the whole number X = (-1)^s m 2^(e - exp + 22), toward zero (|X| < 2^30), and
 // X = sum of d_i 256^i with d_i in -128 .. 127. The rows are laid out as the matrix cores take them: 16-row tile, 64
-// values, digit, then lane 16 q + r's 16 values 16 q .. of row r; rows and values past the ends are zeros. A wave a tile's
+// values, digit, then lane 16 q + r's 16 values 16 q .. of row r; rows and values past the ends are zeros. After the
+// digits, a byte a tile's 64 values: whether any lowest digit is not zero. A wave a tile's
 // 64 values: it reads 128 bytes of each row and writes 4 KB whole. g.lost[row] counts the values that lost bits.
 __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32_t M0, const uint16_t *A1, uint32_t M,
                                                       uint32_t K, HcGrid g, uint8_t *out) {
@@ -173,29 +174,30 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32
   uint8_t *o = out + ((uint64_t)blockIdx.x * nch + ch) * (kHcDigits * 1024) + lane * 16;
 #pragma unroll
   for (uint32_t i = 0; i < kHcDigits; i++) *(uint4 *)(o + 1024 * i) = make_uint4(d[0][i], d[1][i], d[2][i], d[3][i]);
+  const bool low = __any((d[0][0] | d[1][0] | d[2][0] | d[3][0]) != 0u) != 0;
+  if (lane == 0) out[(uint64_t)gridDim.x * nch * (kHcDigits * 1024) + (uint64_t)blockIdx.x * nch + ch] = low ? 1 : 0;
 }
 
-// A row's or token's part of the bound: 2-norm (rounded up), least lsb exponent, and the 2-norm of its lost bits (each
-// less than one of its grid's units, 2^(exp - 156); 0: none).
+// A row's or token's part of the bound: 2-norm (rounded up), the same in units of its values' least lsb (infinite when bits
+// were lost), and the 2-norm of its lost bits (each less than one of its grid's units, 2^(exp - 156); 0: none).
 struct Side {
-  double norm, lost;
-  int lsb, exp;
+  double norm, units, lost;
+  int exp;
 };
 __device__ __forceinline__ Side side_of(const double *norm, const int *lsb, const HcGrid &g, uint32_t i) {
   const uint32_t n = g.lost[i];
   const int e = max(g.exp[i], 1);
-  return {norm[i], n ? ldexp(sqrt((double)n) * 1.0001, e - 156) : 0.0, lsb[i], e};
+  return {norm[i], n ? __builtin_inf() : ldexp(norm[i], -lsb[i]), n ? ldexp(sqrt((double)n) * 1.0001, e - 156) : 0.0, e};
 }
 
 // Whether the digits' sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: no
-// bits lost, every product is a multiple of 2^(r.lsb + t.lsb) and sum|p| <= r.norm t.norm < 2^(r.lsb + t.lsb + 53), so
-// every partial sum of any order is representable and both give the exact sum. Otherwise bounded: the two fp64 values
+// bits lost, every product is a multiple of the two least lsbs' product and sum|p| <= r.norm t.norm is below 2^53 of it, so
+// every partial sum of any order is representable and both give the exact sum (the product of r.units and t.units rounds
+// by 2^-53, which the norms' rounding up covers). Otherwise bounded: the two fp64 values
 // are within bnd, and every value in [v - bnd, v + bnd] rounds to the same fp32.
 __device__ __forceinline__ bool certain(double v, const Side &r, const Side &t, double bound_k) {
-  if (!__builtin_isfinite(v)) return false;
-  const double m = r.norm * t.norm, lost = r.lost * t.norm + r.norm * t.lost;
-  if (lost == 0.0 && r.lsb + t.lsb < 900 && m < ldexp(1.0, r.lsb + t.lsb + 53)) return true;
-  const double bnd = bound_k * m + lost;
+  if (r.units * t.units < 0x1p53) return true;
+  const double bnd = bound_k * (r.norm * t.norm) + (r.lost * t.norm + r.norm * t.lost);
   const float f = (float)v;
   return (float)(v - bnd) == f && (float)(v + bnd) == f;
 }
@@ -212,13 +214,13 @@ __device__ __forceinline__ double diagonals(const int s[kDiagonals]) {
 // parts of cs. A work-group takes 64 rows x 64 tokens, wave w rows 32 (w & 1) .. and tokens 32 (w >> 1) .., as 2 x 2 tiles
 // of 16 x 16, whose digit products of one weight share an accumulator (a part has at most 4096 values: 2^28).
 // The lowest digit is nonzero only for values 2^15 and more below their row's largest (about one in 5000 of a normal
-// row's): a fragment whose lowest digits are all zero skips its products, which leaves 9 of 16 in most chunks.
+// row's): a fragment whose lowest digits are all zero skips their load and products, which leaves 9 of 16 in most chunks.
 // The operands come straight from L2 in the matrix cores' order, the next chunk's while this one's products run.
 // A part keeps to one XCD (nsplit 8), so that each L2 reads one part of both operands; without parts the XCD
 // takes every eighth row tile.
 // kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
 // (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M).
-// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 51 us and up 59, where the fp64 matrix cores took 162 and 141.
+// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 46 us (51 with the lowest digits always loaded) and up 59, where the fp64 matrix cores took 162 and 141.
 template <bool kUp>
 __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
                                                        uint32_t nch, uint32_t nsplit, double *part, float *out32,
@@ -244,16 +246,37 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
 #pragma unroll
       for (uint32_t d = 0; d < kDiagonals; d++) acc[i][j][d] = v4i_t{0, 0, 0, 0};
   v4i_t a[2][kHcDigits], b[2][kHcDigits];
+  // Bit c: chunk c's lowest digits are not all zero (a part has at most 64 chunks). The bytes are read beside the first
+  // chunk's other digits.
+  uint64_t al[2], bl[2];
+  const auto low_digits = [&](uint32_t c, v4i_t (&to)[2][kHcDigits], const uint8_t *const (&from)[2], const uint64_t (&low)[2]) {
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+      if ((low[f] >> c) & 1) to[f][0] = *(const v4i_t *)(from[f] + c * kHcDigits * 1024);
+  };
   const auto load = [&](uint32_t c, v4i_t (&to)[2][kHcDigits], const uint8_t *const (&from)[2]) {
 #pragma unroll
     for (int f = 0; f < 2; f++)
 #pragma unroll
-      for (uint32_t d = 0; d < kHcDigits; d++) to[f][d] = *(const v4i_t *)(from[f] + (c * kHcDigits + d) * 1024);
+      for (uint32_t d = 1; d < kHcDigits; d++) to[f][d] = *(const v4i_t *)(from[f] + (c * kHcDigits + d) * 1024);
   };
-  load(0, a, ap), load(0, b, bp);
+  {
+    const uint8_t *af = A + ((M + 15) / 16) * tile + split * cs, *bf = B + ((N + 15) / 16) * tile + split * cs;
+    const uint32_t c = min(lane, cs - 1);
+    const uint8_t f0 = af[(uint64_t)(m0 / 16) * nch + c], f1 = af[(uint64_t)(m0 / 16 + i1) * nch + c];
+    const uint8_t f2 = bf[(uint64_t)(n0 / 16) * nch + c], f3 = bf[(uint64_t)(n0 / 16 + j1) * nch + c];
+    load(0, a, ap), load(0, b, bp);
+    al[0] = __ballot(f0), al[1] = __ballot(f1), bl[0] = __ballot(f2), bl[1] = __ballot(f3);
+  }
+#pragma unroll
+  for (int f = 0; f < 2; f++) a[f][0] = b[f][0] = v4i_t{0, 0, 0, 0};
+  low_digits(0, a, ap, al), low_digits(0, b, bp, bl);
   for (uint32_t c = 0; c < cs; c++) {
     v4i_t na[2][kHcDigits], nb[2][kHcDigits];
+#pragma unroll
+    for (int f = 0; f < 2; f++) na[f][0] = nb[f][0] = v4i_t{0, 0, 0, 0};
     const uint32_t next = min(c + 1, cs - 1);
+    low_digits(next, na, ap, al), low_digits(next, nb, bp, bl);
     load(next, na, ap), load(next, nb, bp);
 #pragma unroll
     for (uint32_t da = 1; da < kHcDigits; da++)
@@ -264,18 +287,17 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
 #pragma unroll
           for (int j = 0; j < 2; j++)
             acc[i][j][da + db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][da], b[j][db], acc[i][j][da + db], 0, 0, 0);
-    const auto any = [](const v4i_t &v) { return __any((v[0] | v[1] | v[2] | v[3]) != 0) != 0; };
 #pragma unroll
     for (int i = 0; i < 2; i++)
-      if (any(a[i][0]))
+      if ((al[i] >> c) & 1)
 #pragma unroll
         for (uint32_t db = 0; db < kHcDigits; db++)
 #pragma unroll
           for (int j = 0; j < 2; j++)
-            acc[i][j][db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][0], b[j][db], acc[i][j][db], 0, 0, 0);
+            acc[i][j][db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][0], b[j][db], acc[i][j][db], 0, 0, 0);  // (b[j][0] may be zeros)
 #pragma unroll
     for (int j = 0; j < 2; j++)
-      if (any(b[j][0]))
+      if ((bl[j] >> c) & 1)
 #pragma unroll
         for (uint32_t da = 1; da < kHcDigits; da++)
 #pragma unroll

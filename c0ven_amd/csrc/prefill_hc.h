@@ -12,8 +12,8 @@ struct HcShape {
 };
 
 constexpr uint32_t kHcDigits = 4;  // the signed byte digits of a value on its row's or token's grid (moe_prefill_hc.hip)
-// The device bytes of rows x K values' digits: whole 16-row tiles of whole 64-value chunks.
-constexpr uint64_t hc_digit_bytes(uint64_t rows, uint64_t K) { return (rows + 15) / 16 * ((K + 63) / 64) * (kHcDigits * 1024); }
+// The device bytes of rows x K values' digits: whole 16-row tiles of whole 64-value chunks, and a byte each after them.
+constexpr uint64_t hc_digit_bytes(uint64_t rows, uint64_t K) { return (rows + 15) / 16 * ((K + 63) / 64) * (kHcDigits * 1024 + 1); }
 
 // The grids of rows or tokens: the largest exponent field of each one's values and how many of them lose bits on it.
 struct HcGrid {
