@@ -769,6 +769,7 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
         b.nb = c->alloc<uint16_t>(TM * D);
         b.nd = c->alloc<uint8_t>(hc_digit_bytes(TM, D));
         b.ld = c->alloc<uint8_t>(hc_digit_bytes(TM, g.hc_lr));
+        b.wide = c->alloc<uint8_t>((uint64_t)((TM + 31) / 32) * ((g.hc_lr + kHcStreams + 31) / 32));
         for (HcGrid *q : {&b.ng, &b.lg}) q->exp = c->alloc<int>(TM), q->lost = c->alloc<uint32_t>(TM);
         b.ln = c->alloc<double>(TM);
         b.inj = c->alloc<float>(TM * kHcStreams);

@@ -5,10 +5,11 @@
 // sigmoid and mix steps are the same fp32 operations; the two bf16 products (W_down and W_inject against n, W_up
 // against l) are sums of exact products that the decode kernel adds in fp64 in a fixed order and rounds to fp32 once.
 // Here they run on the int8 matrix cores: a row's or token's bf16 values become whole numbers of 2^-29 of its largest
-// value's power of two, in four signed byte digits, and the digits' products add exactly in 32 bits (a value more than
-// 2^22 below the largest loses bits; those are counted). The exact sum, rounded once a K part, is then within
+// value's power of two, in four signed byte digits, and the digits' products add exactly in 32 bits. A value more than
+// 2^22 below the largest loses bits there; where a tile's rows or tokens lose enough of them to leave more than a few sums
+// open, it takes the bf16 values on the fp64 matrix cores instead. Either sum is within
 // (n_mine + n_ref) 2^-53 sum|p| <= (n_mine + n_ref) 2^-53 ||w||_2 ||x||_2 of the fixed order's (Cauchy-Schwarz on the
-// bf16 values; the lost bits add their own term). Where the fp32 rounding of every value in that interval is the same,
+// bf16 values; the digits' lost bits add their own term). Where the fp32 rounding of every value in that interval is the same,
 // it is the fixed order's rounding; and where the products' bits span fewer than 53 (the least lsb of the row's and of
 // the token's values against the Cauchy-Schwarz bound on sum|p|), both sums are exact, whatever their order (ties of
 // fp32 rounding are common for W_up's short sums, and this settles them).
@@ -23,10 +24,12 @@ namespace c0ven {
 namespace {
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
+typedef double v4d_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kHcWG = 256;
 constexpr uint32_t kHcStreams4 = 4;
 constexpr uint32_t kDiagonals = 2 * kHcDigits - 1;  // the digit products' weights: 256^0 .. 256^6
+constexpr uint32_t kGroupK = 128;  // values an fp64 matrix-core chain sums before its sum joins the total
 
 __device__ __forceinline__ uint32_t lane_of() { return threadIdx.x & 63u; }
 
@@ -67,8 +70,8 @@ __device__ __forceinline__ int wg_min(int v, int *red) {
 // arithmetic (each thread's squares in order, then the stream's sum in wg_sum's order; mean rounded to fp32;
 // 1 / sqrtf(mean + 1e-6)): the stream's scale into sc
 // (pf_hc_mix forms n again from R, the scale and gamma), bf16(n) into nb, and the 2-norm (rounded up), least lsb
-// exponent and largest exponent field of bf16(n). Work-group 0 clears the open lists' counts, each its token's counts of
-// values that lose bits. Latency bound (a thread's H / 256 loads, the sum's exchanges): the four streams side by side
+// exponent and largest exponent field of bf16(n). Work-group 0 clears the open lists' counts, each its token's sums of
+// lost bits. Latency bound (a thread's H / 256 loads, the sum's exchanges): the four streams side by side
 // instead of one after another take 23 us at 1000 tokens of H 2560, 39 before.
 __global__ void __launch_bounds__(kHcStreams4 * kHcWG) pf_hc_norm(const float *R, const float *gamma, uint32_t H, float *sc,
                                                                   uint16_t *nb, double *nn, int *nlsb, HcGrid n, HcGrid l,
@@ -133,7 +136,8 @@ __device__ __forceinline__ void transpose4(const uint32_t y[4], uint32_t d[kHcDi
 // X = sum of d_i 256^i with d_i in -128 .. 127. The rows are laid out as the matrix cores take them: 16-row tile, 64
 // values, digit, then lane 16 q + r's 16 values 16 q .. of row r; rows and values past the ends are zeros. After the
 // digits, a byte a tile's 64 values: whether any lowest digit is not zero. A wave a tile's
-// 64 values: it reads 128 bytes of each row and writes 4 KB whole. g.lost[row] counts the values that lost bits.
+// 64 values: it reads 128 bytes of each row and writes 4 KB whole. g.lost[row] receives the lost bits' sum, in
+// 2^-16 of X's units, each rounded up (below 2^31 for K to 32768).
 __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32_t M0, const uint16_t *A1, uint32_t M,
                                                       uint32_t K, HcGrid g, uint8_t *out) {
   const uint32_t nch = (K + 63) / 64, ch = blockIdx.y * (kHcWG / 64) + (threadIdx.x >> 6);
@@ -164,7 +168,8 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32
       const int sh = (int)max(e, 1u) - max(top, 1) + 22;  // (at most 22)
       const uint32_t down = (uint32_t)min(max(-sh, 0), 31);
       const uint32_t x = sh >= 0 ? m << sh : m >> down;
-      lost += (x << down) != m && sh < 0;
+      const uint32_t rest = sh < 0 ? m - (x << down) : 0u;  // (of 2^down)
+      lost += down <= 16 ? rest << (16 - down) : (rest + (1u << (down - 16)) - 1u) >> (down - 16);
       const uint32_t X = (u & 0x8000u) ? 0u - x : x;
       y[i] = (X + 0x00808080u) ^ 0x00808080u;  // each lower byte's digit as a signed byte, its carry in the next
     }
@@ -179,27 +184,46 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32
 }
 
 // A row's or token's part of the bound: 2-norm (rounded up), the same in units of its values' least lsb (infinite when bits
-// were lost), and the 2-norm of its lost bits (each less than one of its grid's units, 2^(exp - 156); 0: none).
+// were lost), the sum of its lost bits, and a power of two above its largest value. wide: its digits are not used.
 struct Side {
-  double norm, units, lost;
-  int exp;
+  double norm, units, lost, top;
 };
-__device__ __forceinline__ Side side_of(const double *norm, const int *lsb, const HcGrid &g, uint32_t i) {
-  const uint32_t n = g.lost[i];
+__device__ __forceinline__ Side side_of(const double *norm, const int *lsb, const HcGrid &g, uint32_t i, bool wide) {
+  const uint32_t n = wide ? 0u : g.lost[i];
   const int e = max(g.exp[i], 1);
-  return {norm[i], n ? __builtin_inf() : ldexp(norm[i], -lsb[i]), n ? ldexp(sqrt((double)n) * 1.0001, e - 156) : 0.0, e};
+  return {norm[i], n ? __builtin_inf() : ldexp(norm[i], -lsb[i]), ldexp((double)n, e - 172), ldexp(1.0, e - 126)};
 }
 
-// Whether the digits' sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: no
-// bits lost, every product is a multiple of the two least lsbs' product and sum|p| <= r.norm t.norm is below 2^53 of it, so
+// Whether the sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: no bits lost,
+// every product is a multiple of the two least lsbs' product and sum|p| <= r.norm t.norm is below 2^53 of it, so
 // every partial sum of any order is representable and both give the exact sum (the product of r.units and t.units rounds
 // by 2^-53, which the norms' rounding up covers). Otherwise bounded: the two fp64 values
 // are within bnd, and every value in [v - bnd, v + bnd] rounds to the same fp32.
 __device__ __forceinline__ bool certain(double v, const Side &r, const Side &t, double bound_k) {
   if (r.units * t.units < 0x1p53) return true;
-  const double bnd = bound_k * (r.norm * t.norm) + (r.lost * t.norm + r.norm * t.lost);
+  const double bnd = bound_k * (r.norm * t.norm) + (r.lost * t.top + r.top * t.lost);
   const float f = (float)v;
   return (float)(v - bnd) == f && (float)(v + bnd) == f;
+}
+
+// Whether a wave's 32 rows and 32 tokens take wide_products: their lost bits would leave more than about 3% of the sums
+// open. A sum is about r.norm t.norm / sqrt(K), half its fp32 unit 2^-25 of that; limit is 2^-30 / sqrt(K), against the
+// lost term over the norms. A normal row of 10240 loses bits in one value of 0.8% of the rows, 4 to 8 times less than the limit.
+__device__ __forceinline__ bool tile_is_wide(const double *rn, const double *tn, const HcGrid &gr, const HcGrid &gt,
+                                             uint32_t M, uint32_t N, uint32_t m0, uint32_t n0, double limit) {
+  const uint32_t lane = lane_of(), f32 = lane % 32;
+  const bool row = lane < 32;  // lanes 0-31 the rows, 32-63 the tokens
+  const uint32_t i = row ? min(m0 + f32, M - 1) : min(n0 + f32, N - 1);
+  const uint32_t n = (row ? gr.lost : gt.lost)[i];
+  if (!__any(n != 0u)) return false;
+  const int e = max((row ? gr.exp : gt.exp)[i], 1);
+  const double norm = (row ? rn : tn)[i];
+  // (Both far inside fp32's range; a zero row has neither part.)
+  float lost = norm == 0.0 ? 0.0f : (float)(ldexp((double)n, e - 172) / norm), top = norm == 0.0 ? 0.0f : (float)(ldexp(1.0, e - 126) / norm);
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) lost = fmaxf(lost, __shfl_xor(lost, o, 64)), top = fmaxf(top, __shfl_xor(top, o, 64));
+  const float other = __shfl_xor(top, 32, 64);
+  return __any((double)lost * other > limit) != 0;
 }
 
 // sum of s[i] 256^i, rounded to fp64 once: a part has at most 4096 values, so |s[6]| <= 2^24, |s[5]| <= 2^26, |s[4]| <= 2^27,
@@ -210,31 +234,77 @@ __device__ __forceinline__ double diagonals(const int s[kDiagonals]) {
   return __builtin_fma(__builtin_fma(p, 65536.0, q), 0x1p24, r);
 }
 
-// C = A B^T over the digits of the rows (M of them, A) and of the tokens (N, B), nch 64-value chunks in blockIdx.x % nsplit
-// parts of cs. A work-group takes 64 rows x 64 tokens, wave w rows 32 (w & 1) .. and tokens 32 (w >> 1) .., as 2 x 2 tiles
-// of 16 x 16, whose digit products of one weight share an accumulator (a part has at most 4096 values: 2^28).
-// The lowest digit is nonzero only for values 2^15 and more below their row's largest (about one in 5000 of a normal
-// row's): a fragment whose lowest digits are all zero skips their load and products, which leaves 9 of 16 in most chunks.
-// The operands come straight from L2 in the matrix cores' order, the next chunk's while this one's products run.
-// A part keeps to one XCD (nsplit 8), so that each L2 reads one part of both operands; without parts the XCD
-// takes every eighth row tile.
-// kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
-// (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M).
-// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 46 us (51 with the lowest digits always loaded) and up 59, where the fp64 matrix cores took 162 and 141.
-template <bool kUp>
-__global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
-                                                       uint32_t nch, uint32_t nsplit, double *part, float *out32,
-                                                       const double *rn, const double *tn, const int *rl,
-                                                       const int *tl, HcGrid gr, HcGrid gt, double bound_k,
-                                                       uint32_t *open, uint32_t *cnt) {
-  const uint32_t nmt = (M + 63) / 64, split = blockIdx.x % nsplit, item = blockIdx.x / nsplit;
-  const uint32_t mt = item % nmt, nt = item / nmt, cs = nch / nsplit;
-  const uint32_t lane = lane_of(), w = threadIdx.x >> 6, g = lane / 16, c16 = lane % 16;
-  const uint32_t m0 = 64 * mt + 32 * (w & 1), n0 = 64 * nt + 32 * (w >> 1);
-  // 16 x 16 tiles wholly past the rows or the tokens are skipped: a wave with none returns (the kernel has no barrier),
-  // the others repeat their first tile's operands and drop its sums.
-  if (m0 >= M || n0 >= N) return;
-  const uint32_t i1 = m0 + 16 < M ? 1u : 0u, j1 = n0 + 16 < N ? 1u : 0u;
+// The sums of a wave's 32 rows and 32 tokens over K range kb .. ke from the bf16 values (rows of A0's first M0, then A1's) on
+// the fp64 matrix cores. Lane l (g = l / 16) holds values 8 g .. 8 g + 7 of a 32-value step of both operands, step m of the
+// matrix instruction its m'th (the order of a sum is free here: the bound covers any); the A operand's lane c takes row
+// 4 (c % 4) + c / 4, so that v[i][j][q] is digit_products' element. Each kGroupK values' chain starts from zero and is added
+// to the total.
+__device__ __forceinline__ void wide_products(const uint16_t *A0, uint32_t M0, const uint16_t *A1, uint32_t M,
+                                              const uint16_t *B, uint32_t N, uint32_t K, uint32_t kb, uint32_t ke,
+                                              uint32_t m0, uint32_t n0, double (&v)[2][2][4]) {
+  const uint32_t lane = lane_of(), g = lane / 16, c16 = lane % 16;
+  const uint16_t *ar[2], *br[2];
+#pragma unroll
+  for (int f = 0; f < 2; f++) {
+    const uint32_t row = min(m0 + 16 * f + 4 * (c16 % 4) + c16 / 4, M - 1), tok = min(n0 + 16 * f + c16, N - 1);
+    ar[f] = row < M0 ? A0 + (uint64_t)row * K : A1 + (uint64_t)(row - M0) * K;
+    br[f] = B + (uint64_t)tok * K;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[i][j][q] = 0.0;
+  for (uint32_t kg = kb; kg < ke; kg += kGroupK) {
+    v4d_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] = v4d_t{0.0, 0.0, 0.0, 0.0};
+    const uint32_t kge = min(ke, kg + kGroupK);
+    for (uint32_t kc = kg; kc < kge; kc += 32) {
+      const uint32_t k = kc + 8 * g;
+      const bool ok = k < kge;  // (K is a multiple of 8: a lane's eight values are all in or all out)
+      uint32_t a[2][4], b[2][4];
+#pragma unroll
+      for (int f = 0; f < 2; f++) {
+        const uint4 x = ok ? *(const uint4 *)(ar[f] + k) : make_uint4(0u, 0u, 0u, 0u);
+        const uint4 y = ok ? *(const uint4 *)(br[f] + k) : make_uint4(0u, 0u, 0u, 0u);
+        a[f][0] = x.x, a[f][1] = x.y, a[f][2] = x.z, a[f][3] = x.w;
+        b[f][0] = y.x, b[f][1] = y.y, b[f][2] = y.z, b[f][3] = y.w;
+      }
+#pragma unroll
+      for (int m = 0; m < 8; m++) {
+        double ad[2], bd[2];
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+          ad[f] = m % 2 ? bf16_hi(a[f][m / 2]) : bf16_lo(a[f][m / 2]);
+          bd[f] = m % 2 ? bf16_hi(b[f][m / 2]) : bf16_lo(b[f][m / 2]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[i], bd[j], acc[i][j], 0, 0, 0);
+      }
+    }
+    // (The f64 form's result layout: element q of lane l is A lane 4 q + l / 16's row, B lane l % 16's token.)
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[i][j][q] = __dadd_rn(v[i][j][q], acc[i][j][q]);
+  }
+}
+
+// The same from the digits of part `split` (cs of nch 64-value chunks): each sum exact in 32-bit diagonals, rounded once.
+// v[i][j][q]: row m0 + 16 i + 4 g + q, token n0 + 16 j + c16 (g = lane / 16, c16 = lane % 16); i1, j1: 0 where the second
+// tile lies wholly past the rows or tokens (the first's operands are repeated and its sums dropped).
+__device__ __forceinline__ void digit_products(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N, uint32_t nch,
+                                               uint32_t split, uint32_t cs, uint32_t m0, uint32_t n0, uint32_t i1,
+                                               uint32_t j1, const HcGrid &gr, const HcGrid &gt, double (&v)[2][2][4]) {
+  const uint32_t lane = lane_of(), g = lane / 16, c16 = lane % 16;
   const uint64_t tile = (uint64_t)nch * (kHcDigits * 1024), first = (uint64_t)split * cs * (kHcDigits * 1024) + lane * 16;
   const uint8_t *ap[2] = {A + m0 / 16 * tile + first, A + (m0 / 16 + i1) * tile + first};
   const uint8_t *bp[2] = {B + n0 / 16 * tile + first, B + (n0 / 16 + j1) * tile + first};
@@ -308,47 +378,92 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
 #pragma unroll
       for (uint32_t d = 0; d < kHcDigits; d++) a[f][d] = na[f][d], b[f][d] = nb[f][d];
   }
-  // acc[i][j][.][q]: row m0 + 16 i + 4 g + q, token n0 + 16 j + c16. (M is a multiple of 4.)
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const uint32_t row = m0 + 16 * i + 4 * g;
-    if (row >= M) continue;
-    Side rs[4];
+    const uint32_t row = min(m0 + 16 * i + 4 * g, M - 4);  // (M is a multiple of 4)
+    int er[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      if constexpr (kUp)
-        rs[q] = side_of(rn, rl, gr, row + q);
-      else
-        rs[q].exp = max(gr.exp[row + q], 1);
-    }
+    for (int q = 0; q < 4; q++) er[q] = max(gr.exp[row + q], 1);
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const uint32_t tok = n0 + 16 * j + c16;
-      if (tok >= N) continue;
-      Side ts;
-      if constexpr (kUp)
-        ts = side_of(tn, tl, gt, tok);
-      else
-        ts.exp = max(gt.exp[tok], 1);
-      double v[4];
+      const int et = max(gt.exp[min(n0 + 16 * j + c16, N - 1)], 1) - 312;
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         int s[kDiagonals];
 #pragma unroll
         for (uint32_t d = 0; d < kDiagonals; d++) s[d] = acc[i][j][d][q];
-        v[q] = ldexp(diagonals(s), rs[q].exp + ts.exp - 312);
+        v[i][j][q] = ldexp(diagonals(s), er[q] + et);
       }
+    }
+  }
+}
+
+// C = A B^T over the digits of the rows (M of them, A) and of the tokens (N, B), nch 64-value chunks in blockIdx.x % nsplit
+// parts of cs. A work-group takes 64 rows x 64 tokens, wave w rows 32 (w & 1) .. and tokens 32 (w >> 1) .., as 2 x 2 tiles
+// of 16 x 16, whose digit products of one weight share an accumulator (a part has at most 4096 values: 2^28).
+// The lowest digit is nonzero only for values 2^15 and more below their row's largest (about one in 5000 of a normal
+// row's): a fragment whose lowest digits are all zero skips their load and products, which leaves 9 of 16 in most chunks.
+// The operands come straight from L2 in the matrix cores' order, the next chunk's while this one's products run.
+// A part keeps to one XCD (nsplit 8), so that each L2 reads one part of both operands; without parts the XCD
+// takes every eighth row tile.
+// A wave whose rows or tokens lost too many bits (tile_is_wide) takes their bf16 values (A0's first M0 rows, then A1's; Bb; K a
+// row) on the fp64 matrix cores. With the digits for those too, nearly every sum of such a token was left open, and the
+// fixed-order kernels took most of the step: 1000 tokens of H 2560 with two channels 3000 times the others, the whole
+// step 2.0 ms (3.7 with W_down eight times as large), 0.70 (0.80) with this, 0.96 with all products in fp64; 0.58 on normal
+// values either way.
+// kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
+// (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M), and
+// whether a 32 x 32 tile was wide to wide_map (token tiles x row tiles).
+// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 46 us (51 with the lowest digits always loaded) and up 59, where the fp64 matrix cores took 162 and 141.
+template <bool kUp>
+__global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
+                                                       const uint16_t *A0, uint32_t M0, const uint16_t *A1,
+                                                       const uint16_t *Bb, uint32_t K, uint32_t nch, uint32_t nsplit,
+                                                       double *part, float *out32, uint8_t *wide_map, const double *rn,
+                                                       const double *tn, const int *rl, const int *tl, HcGrid gr,
+                                                       HcGrid gt, double limit, double bound_digits, double bound_wide,
+                                                       uint32_t *open, uint32_t *cnt) {
+  const uint32_t nmt = (M + 63) / 64, split = blockIdx.x % nsplit, item = blockIdx.x / nsplit;
+  const uint32_t mt = item % nmt, nt = item / nmt, cs = nch / nsplit;
+  const uint32_t lane = lane_of(), w = threadIdx.x >> 6, g = lane / 16, c16 = lane % 16;
+  const uint32_t m0 = 64 * mt + 32 * (w & 1), n0 = 64 * nt + 32 * (w >> 1);
+  // 16 x 16 tiles wholly past the rows or the tokens are skipped: a wave with none returns (the kernel has no barrier),
+  // the others repeat their first tile's operands and drop its sums.
+  if (m0 >= M || n0 >= N) return;
+  const uint32_t i1 = m0 + 16 < M ? 1u : 0u, j1 = n0 + 16 < N ? 1u : 0u;
+  const bool wide = tile_is_wide(rn, tn, gr, gt, M, N, m0, n0, limit);
+  if (!kUp && split == 0 && lane == 0) wide_map[n0 / 32 * ((M + 31) / 32) + m0 / 32] = wide ? 1 : 0;
+  const double bound_k = wide ? bound_wide : bound_digits;
+  double v[2][2][4];
+  if (wide)
+    wide_products(A0, M0, A1, M, Bb, N, K, 64 * split * cs, min(K, 64 * (split + 1) * cs), m0, n0, v);
+  else
+    digit_products(A, M, B, N, nch, split, cs, m0, n0, i1, j1, gr, gt, v);
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t row = m0 + 16 * i + 4 * g;
+    if (row >= M) continue;
+    Side rs[4];
+    if constexpr (kUp)
+#pragma unroll
+      for (int q = 0; q < 4; q++) rs[q] = side_of(rn, rl, gr, row + q, wide);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const uint32_t tok = n0 + 16 * j + c16;
+      if (tok >= N) continue;
       if constexpr (kUp) {
-        *(float4 *)(out32 + (uint64_t)tok * M + row) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+        const Side ts = side_of(tn, tl, gt, tok, wide);
+        *(float4 *)(out32 + (uint64_t)tok * M + row) =
+            make_float4((float)v[i][j][0], (float)v[i][j][1], (float)v[i][j][2], (float)v[i][j][3]);
 #pragma unroll
         for (int q = 0; q < 4; q++)
-          if (!certain(v[q], rs[q], ts, bound_k)) {  // open: pf_hc_up_fix writes it
+          if (!certain(v[i][j][q], rs[q], ts, bound_k)) {  // open: pf_hc_up_fix writes it
             const uint32_t at = atomicAdd(cnt, 1u);
             open[2 * at] = tok, open[2 * at + 1] = row + q;
           }
       } else {
         double *o = part + ((uint64_t)split * N + tok) * M + row;
-        *(double2 *)o = make_double2(v[0], v[1]), *(double2 *)(o + 2) = make_double2(v[2], v[3]);
+        *(double2 *)o = make_double2(v[i][j][0], v[i][j][1]), *(double2 *)(o + 2) = make_double2(v[i][j][2], v[i][j][3]);
       }
     }
   }
@@ -359,14 +474,15 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
 // raw entry is written by pf_hc_down_fix). force_open sends all.
 __global__ void __launch_bounds__(kHcWG) pf_hc_down_fin(const double *part, uint32_t T, uint32_t M, uint32_t nsplit,
                                                         const double *rn, const double *tn, const int *rl,
-                                                        const int *tl, HcGrid gr, HcGrid gt, double bound_k,
-                                                        bool force_open, float *raw, uint32_t *open, uint32_t *cnt) {
+                                                        const int *tl, HcGrid gr, HcGrid gt, const uint8_t *wide_map,
+                                                        double bound_digits, double bound_wide, bool force_open,
+                                                        float *raw, uint32_t *open, uint32_t *cnt) {
   const uint32_t t = blockIdx.x;
-  const Side ts = side_of(tn, tl, gt, t);
   for (uint32_t row = threadIdx.x; row < M; row += kHcWG) {
     double v = 0.0;
     for (uint32_t s = 0; s < nsplit; s++) v = __dadd_rn(v, part[((uint64_t)s * T + t) * M + row]);
-    if (!force_open && certain(v, side_of(rn, rl, gr, row), ts, bound_k)) {
+    const bool wide = wide_map[t / 32 * ((M + 31) / 32) + row / 32] != 0;
+    if (!force_open && certain(v, side_of(rn, rl, gr, row, wide), side_of(tn, tl, gt, t, wide), wide ? bound_wide : bound_digits)) {
       raw[(uint64_t)t * M + row] = (float)v;
     } else {
       const uint32_t at = atomicAdd(cnt, 1u);
@@ -547,23 +663,25 @@ hipError_t prefill_hc_pre(const HcShape &S, const HcLayer &L, const HcBufs &b, c
   const uint32_t nd = D / 64, nu = (lr + 63) / 64, tiles = (T + 15) / 16;
   pf_hc_norm<<<T, kHcStreams4 * kHcWG, 0, st>>>(R, L.gamma, H, b.sc, b.nb, b.nn, b.nlsb, b.ng, b.lg, b.cnt);
   pf_hc_digits<<<dim3(tiles, (nd + 3) / 4), kHcWG, 0, st>>>(b.nb, T, nullptr, T, D, b.ng, b.nd);
-  // The down GEMM: K = 4H in kHcDownSplit parts. Roundings on a sum's path: here one a part and one a part's addition; in
-  // the fixed order 8 (chain) + 1 + 3 (tree) + K / 2048 (the slot's chunks) + 16 (the slots); doubled, and 2^-53 each.
-  const double bd = 2.0 * (1.0 + kHcDownSplit + 28.0 + D / 2048.0);
+  // The down GEMM: K = 4H in kHcDownSplit parts. Roundings on a sum's path: here one a part (wide: at most kGroupK of a
+  // matrix-core chain and one a group's total) and one a part's addition; in the fixed order 8 (chain) + 1 + 3 (tree) +
+  // K / 2048 (the slot's chunks) + 16 (the slots); doubled, and 2^-53 each.
+  const double nd_ref = kHcDownSplit + 28.0 + D / 2048.0, bd = 2.0 * (1.0 + nd_ref) * 0x1p-53;
+  const double bdw = 2.0 * (kGroupK + D / kHcDownSplit / kGroupK + 1.0 + nd_ref) * 0x1p-53;
   pf_hc_gemm<false><<<(Md + 63) / 64 * ((T + 63) / 64) * kHcDownSplit, kHcWG, 0, st>>>(
-      L.dig_down, Md, b.nd, T, nd, kHcDownSplit, b.part, nullptr, nullptr, nullptr, nullptr, nullptr, L.grid, b.ng, 0.0, nullptr,
-      nullptr);
-  pf_hc_down_fin<<<T, kHcWG, 0, st>>>(b.part, T, Md, kHcDownSplit, L.row_norm, b.nn, L.row_lsb, b.nlsb, L.grid, b.ng,
-                                      bd * 0x1p-53, force_open, b.raw, b.open, b.cnt);
+      L.dig_down, Md, b.nd, T, L.w_down, lr, L.w_inj, b.nb, D, nd, kHcDownSplit, b.part, nullptr, b.wide, L.row_norm, b.nn,
+      nullptr, nullptr, L.grid, b.ng, 0x1p-30 / sqrt((double)D), 0.0, 0.0, nullptr, nullptr);
+  pf_hc_down_fin<<<T, kHcWG, 0, st>>>(b.part, T, Md, kHcDownSplit, L.row_norm, b.nn, L.row_lsb, b.nlsb, L.grid, b.ng, b.wide,
+                                      bd, bdw, force_open, b.raw, b.open, b.cnt);
   pf_hc_down_fix<<<1024, kHcWG, 0, st>>>(L.w_down, L.w_inj, lr, D, b.nb, b.open, b.cnt, b.raw);
   pf_hc_down_epi<<<T, kHcWG, 0, st>>>(b.raw, lr, b.lb, b.inj, b.ln, b.llsb, b.lg);
   // The up GEMM: 4H rows of W_up against bf16(l), K = lr; the fixed order is a k chain of lr terms.
   pf_hc_digits<<<dim3(tiles, (nu + 3) / 4), kHcWG, 0, st>>>(b.lb, T, nullptr, T, lr, b.lg, b.ld);
-  const double bu = 2.0 * (1.0 + 1.0 + lr);
+  const double bu = 2.0 * (1.0 + 1.0 + lr) * 0x1p-53, buw = 2.0 * (kGroupK + lr / kGroupK + 1.0 + lr) * 0x1p-53;
   const HcGrid gu{L.grid.exp + Md, L.grid.lost + Md};
-  pf_hc_gemm<true><<<(D + 63) / 64 * ((T + 63) / 64), kHcWG, 0, st>>>(L.dig_up, D, b.ld, T, nu, 1, nullptr, b.a,
-                                                                      L.row_norm + Md, b.ln, L.row_lsb + Md, b.llsb, gu, b.lg,
-                                                                      bu * 0x1p-53, b.open_up, b.cnt + 1);
+  pf_hc_gemm<true><<<(D + 63) / 64 * ((T + 63) / 64), kHcWG, 0, st>>>(
+      L.dig_up, D, b.ld, T, L.w_up, D, nullptr, b.lb, lr, nu, 1, nullptr, b.a, nullptr, L.row_norm + Md, b.ln,
+      L.row_lsb + Md, b.llsb, gu, b.lg, 0x1p-30 / sqrt((double)lr), bu, buw, b.open_up, b.cnt + 1);
   pf_hc_up_fix<<<256, kHcWG, 0, st>>>(L.w_up, lr, D, b.lb, b.open_up, b.cnt + 1, b.a);
   const uint64_t nx = (uint64_t)T * H;
   pf_hc_mix<<<(uint32_t)((nx + 2 * kHcWG - 1) / (2 * kHcWG)), kHcWG, 0, st>>>(R, L.gamma, b.sc, b.a, T, H, b.x);

@@ -15,7 +15,8 @@ constexpr uint32_t kHcDigits = 4;  // the signed byte digits of a value on its r
 // The device bytes of rows x K values' digits: whole 16-row tiles of whole 64-value chunks, and a byte each after them.
 constexpr uint64_t hc_digit_bytes(uint64_t rows, uint64_t K) { return (rows + 15) / 16 * ((K + 63) / 64) * (kHcDigits * 1024 + 1); }
 
-// The grids of rows or tokens: the largest exponent field of each one's values and how many of them lose bits on it.
+// The grids of rows or tokens: the largest exponent field of each one's values, and the sum of the bits they lose on that
+// grid (pf_hc_digits).
 struct HcGrid {
   int *exp;
   uint32_t *lost;
@@ -43,6 +44,7 @@ struct HcBufs {
   float *sc, *raw, *inj, *a, *x;
   uint16_t *nb, *lb;  // bf16(n), bf16(l)
   uint8_t *nd, *ld;   // their digits: the GEMMs' operands
+  uint8_t *wide;      // which 32 x 32 tiles of the down GEMM did not take the digits
   HcGrid ng, lg;
   double *nn, *ln, *part;
   int *nlsb, *llsb;  // the least lsb exponent of each token's bf16(n), bf16(l)

@@ -2,6 +2,7 @@
 1.1-1.2; model.cpp:1350-1416 runs them as separate kernels) against the oracle's mix, block and combine, bit for bit:
 the updated streams R, y, the routing."""
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -123,3 +124,60 @@ def test_forward_hc_prefill_wide_values(lr, T):
     assert np.array_equal(ids, io) and np.array_equal(w, wo)
     assert np.array_equal(y, yo), h.max_abs(y, yo)
     assert np.array_equal(R2, Ro), h.max_abs(R2, Ro)
+
+
+def test_forward_hc_prefill_not_finite():
+    """Tokens with infinities and NaN among finite ones, and a row of W_down with an infinity: as the oracle's, NaN where it has
+    one (the payload aside)."""
+    H, F, E, K, lr, T = 512, 256, 32, 4, 64, 40
+    say("forward_hc prefill, not finite")
+    L = h.Layer(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, moe.QT_Q8_0, moe.QT_Q8_0, seed=3, zipf=1.1)
+    hc = h.HcModule(H, lr, seed=14)
+    hc.down[7, 5] = 0x7F80
+    blk = moe.MoeBlock(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, True, moe.QT_Q8_0, moe.QT_Q8_0, n_layer=1, max_tokens=T,
+                       hc_lr=lr, exact_router=True)
+    L.upload(blk, 0)
+    hc.load(blk, 0)
+    r = np.random.default_rng(15)
+    R = r.standard_normal((T, 4, H)).astype(np.float32)
+    R[2, 1, 9], R[17, 0, 3], R[33, 3, 100] = np.inf, -np.inf, np.nan
+    R[20, :, 5] = 0.0  # (0 times the infinite weight)
+    x, inj = hc.pre(R)
+    fine = np.isfinite(x).all(1)
+    assert fine.sum() > 8 and not fine.all()
+    R2, y, _, _ = blk.forward_hc(0, R)
+    yo, _, _ = L.oracle_forward(np.where(fine[:, None], x, np.float32(0)))
+    Ro = h.HcModule.post(R, inj, np.where(fine[:, None], yo, y))
+    blk.close()
+    assert np.array_equal(y[fine], yo[fine])
+    assert np.array_equal(R2[fine], Ro[fine], equal_nan=True)
+
+
+def test_forward_hc_prefill_outliers_cost():
+    """A step whose tokens have a few channels thousands of times the others (values that lose bits of the digits' grid) leaves
+    no more sums to the fixed-order kernels than another: it took 3.5 times as long while it did, and takes at most twice
+    (the products then run on the fp64 matrix cores)."""
+    H, F, E, K, lr, T = 2560, 640, 16, 2, 320, 1000
+    say("forward_hc prefill outliers cost")
+    L = h.Layer(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, moe.QT_Q8_0, moe.QT_Q8_0, seed=5, experts=[0])
+    hc = h.HcModule(H, lr, seed=16)
+    blk = moe.MoeBlock(H, F, E, K, moe.QT_Q4_K, moe.QT_Q8_0, True, moe.QT_Q8_0, moe.QT_Q8_0, n_layer=1, max_tokens=T, hc_lr=lr)
+    L.upload(blk, 0)
+    hc.load(blk, 0)
+    R = np.random.default_rng(17).standard_normal((T, 4, H)).astype(np.float32)
+    us = []
+    for scale in (1.0, 3000.0):
+        R[:, :, [11, 1500]] *= np.float32(scale)
+        d = h.Dev()
+        Rd, y = d.put(R), d.alloc(T * H * 4)
+        best = []
+        for _ in range(12):
+            t0 = time.perf_counter()
+            blk.forward_hc_async(0, Rd, T, y)
+            blk.sync()
+            best.append(time.perf_counter() - t0)
+        d.free()
+        us.append(min(best) * 1e6)
+    blk.close()
+    say("us", us)
+    assert us[1] <= 2.0 * us[0], us
