@@ -608,7 +608,8 @@ __global__ void __launch_bounds__(kPfWG) pf_topk_cert(float *logits, const uint1
 //   the masks  built by pf_topk as it selects (global atomics on masks the router's gate-row work-groups cleared),
 //              or, for pre-routed ids, by pf_masks (one work-group a window, LDS atomics, written out whole);
 //   pf_place   one work-group a window: the counts, the experts' bases and the window's starts from the masks, then
-//              position = start of (window, expert) + the lower bits of the mask; perm and inv; the MoeTile records.
+//              position = start of (window, expert) + the lower bits of the mask; perm and inv; three more: the MoeTile
+//              records and the span lists.
 
 constexpr uint32_t kDispWG = 512;
 
@@ -643,9 +644,11 @@ __device__ __forceinline__ uint32_t block_scan512(uint32_t v, uint32_t *wsum) {
   return v + add;
 }
 
-// The span lists pf_place writes beside the tiles: positions a span (0: none; at most 16 kSpanClasses), the records,
-// their counts. The longest spans come first, so that the last work-groups of a launch are short ones.
-constexpr uint32_t kSpanClasses = 16;
+// The span lists pf_place writes beside the tiles: positions a span (0: none), the records, their counts. The experts with
+// the most positions come first (in classes of 16 positions), so that the last work-groups of a launch are short ones;
+// an expert's spans are neighbours, so that they read its weights at one time (4096 tokens of Q4_K over 512 experts
+// evenly, 80 positions an expert: gate/up 341 us with all whole spans before all rests, 327 this way).
+constexpr uint32_t kSpanClasses = 64;
 struct PfSpans {
   uint32_t len[2];
   MoeTile *list[2];
@@ -657,14 +660,16 @@ constexpr uint32_t kScanBatch = 32;  // window masks a thread holds at once (all
 // One work-group a window. Thread e counts expert e's assignments in every window (the masks' popcounts, all loaded
 // before the first is used) and in the windows before this one; a scan over experts gives each expert's base, so the
 // (window, expert) start is base + the earlier windows' count. The window's assignments are then placed at that start
-// plus the popcount of the lower mask bits; window 0's work-group also writes the MoeTile records (at most MOE_TILE
-// rows) and their count.
+// plus the popcount of the lower mask bits. Three work-groups past the windows' write the MoeTile records (at most MOE_TILE
+// rows, in expert order) and the span lists, with their counts (with all of them in window 0's work-group before its
+// placing, the launch took 17.0 us at 2048 tokens and two lists between its events, 13.5 this way).
 __global__ void __launch_bounds__(kDispWG) pf_place(const int32_t *ids, uint32_t T, uint32_t K, uint32_t E,
                                                     uint32_t nwin, const unsigned long long *masks, MoeTile *tiles,
                                                     uint32_t *ntiles, uint32_t *perm, uint32_t *inv, PfSpans sp) {
-  __shared__ uint32_t wsum[kDispWG / 64], start[kDispWG], hist[kSpanClasses + 2];
+  __shared__ uint32_t wsum[kDispWG / 64], start[kDispWG], hist[kSpanClasses];
   __shared__ unsigned long long mine[kDispWG];
   const uint32_t w = blockIdx.x, e = threadIdx.x, ec = min(e, E - 1);
+  if (w > nwin && sp.len[w - nwin - 1] == 0) return;
   uint32_t c = 0, before = 0;
   for (uint32_t j0 = 0; j0 < nwin; j0 += kScanBatch) {
     // Unconditional loads (clamped indices, masked after), so that all are in flight before the first is used.
@@ -679,9 +684,7 @@ __global__ void __launch_bounds__(kDispWG) pf_place(const int32_t *ids, uint32_t
     }
   }
   const uint32_t base = block_scan512(c, wsum) - c;
-  start[e] = base + before;
-  mine[e] = e < E ? masks[(uint64_t)w * E + e] : 0ull;
-  if (w == 0) {
+  if (w == nwin) {
     const uint32_t nt = (c + MOE_TILE - 1) / MOE_TILE, t0 = block_scan512(nt, wsum) - nt;
     if (e < E)
       for (uint32_t i = 0; i < nt; i++) {
@@ -690,33 +693,37 @@ __global__ void __launch_bounds__(kDispWG) pf_place(const int32_t *ids, uint32_t
         tiles[t0 + i] = m;
       }
     if (e == E - 1) *ntiles = t0 + nt;
-#pragma unroll
-    for (uint32_t v = 0; v < 2; v++) {  // the same positions in the GEMMs' spans, the longest first
-      const uint32_t P = sp.len[v];
-      if (P == 0) continue;
-      const uint32_t full = c / P, rem = c % P, k = (rem + 15) / 16;  // whole spans, then the rest by position tiles
-      const uint32_t f0 = block_scan512(full, wsum) - full;
-      if (e < kSpanClasses + 1) hist[e] = 0u;
-      if (e == kDispWG - 1) hist[kSpanClasses + 1] = f0 + full;  // all whole spans
-      __syncthreads();
-      const uint32_t at = rem ? atomicAdd(&hist[k], 1u) : 0u;
-      __syncthreads();
-      uint32_t before_k = hist[kSpanClasses + 1], all = before_k;
-      for (uint32_t i = 1; i <= kSpanClasses; i++) all += hist[i], before_k += i > k ? hist[i] : 0u;
-      if (e < E) {
-        MoeTile m;
-        m.expert = e, m.slot = e, m.count = P;
-        for (uint32_t i = 0; i < full; i++) {
-          m.start = base + P * i;
-          sp.list[v][f0 + i] = m;
-        }
-        m.start = base + P * full, m.count = rem;
-        if (rem) sp.list[v][before_k + at] = m;
-      }
-      if (e == 0) sp.n[v] = all;
-      __syncthreads();
-    }
+    return;
   }
+  if (w > nwin) {  // the same positions in a GEMM's spans
+    const uint32_t v = w - nwin - 1, P = sp.len[v], ns = (c + P - 1) / P;
+    const uint32_t k = kSpanClasses - min((c + 15) / 16, kSpanClasses);  // the expert's class, the fullest first
+    if (e < kSpanClasses) hist[e] = 0u;
+    __syncthreads();
+    uint32_t at = ns ? atomicAdd(&hist[k], ns) : 0u;
+    __syncthreads();
+    if (e < kSpanClasses) {  // (one wave) the classes' starts
+      const uint32_t n = hist[e];
+      uint32_t x = n;
+#pragma unroll
+      for (uint32_t o = 1; o < kSpanClasses; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (e >= o) x += y;
+      }
+      hist[e] = x - n;
+      if (e == kSpanClasses - 1) sp.n[v] = x;
+    }
+    __syncthreads();
+    if (ns) at += hist[k];
+    for (uint32_t i = 0; i < ns; i++) {
+      MoeTile m;
+      m.expert = e, m.slot = e, m.start = base + P * i, m.count = min(P, c - P * i);
+      sp.list[v][at + i] = m;
+    }
+    return;
+  }
+  start[e] = base + before;
+  mine[e] = e < E ? masks[(uint64_t)w * E + e] : 0ull;
   __syncthreads();
   const uint32_t t0 = 64 * w, a0 = t0 * K, a1 = min(T, t0 + 64) * K;
   for (uint32_t a = a0 + e; a < a1; a += kDispWG) {
@@ -1453,12 +1460,14 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
     }
 }
 
-// Work-group b of a span launch: span *sp's row group *rb (nrb a span). XCD x (b % 8) takes spans x, x + 8, ..., a span's
-// row groups one after another, so a span's activations are read into one XCD's L2 and, the list being longest first, the
-// XCDs get equal work. The grid is span_grid(most spans, nrb); false past the last span.
+// Work-group b of a span launch: span *sp's row group *rb (nrb a span). XCD x (b % 8) takes one span of every eight, its row
+// groups one after another, so a span's activations are read into one XCD's L2; which of the eight moves on by one from
+// eight to eight, as an expert's spans are neighbours and its last one is shorter (two an expert and no move: every rest
+// on the odd XCDs, gate/up 375 us instead of 327 at 80 positions an expert). The grid is span_grid(most spans, nrb); false
+// past the last span.
 __device__ __forceinline__ bool span_item(uint32_t b, uint32_t nrb, uint32_t nspans, uint32_t *sp, uint32_t *rb) {
-  const uint32_t j = b / 8;
-  *sp = (j / nrb) * 8 + b % 8, *rb = j % nrb;
+  const uint32_t j = b / 8, r = j / nrb;
+  *sp = r * 8 + (b + r) % 8, *rb = j % nrb;
   return *sp < nspans;
 }
 constexpr uint32_t span_grid(uint32_t spans, uint32_t nrb) { return (spans + 7) / 8 * 8 * nrb; }
@@ -1696,7 +1705,7 @@ hipError_t routed_experts(const PfShape &S, const PfLayer &L, const PfBufs &b, h
     HookScope k(hook, "pf_dispatch", st);
     const uint32_t nwin = pf_windows(T);
     if (!masks_built) pf_masks<<<nwin, kDispWG, 0, st>>>(b.ids, T, K, E, b.masks);
-    pf_place<<<nwin, kDispWG, 0, st>>>(b.ids, T, K, E, nwin, b.masks, b.tiles, b.ntiles, b.perm, b.inv, sp);
+    pf_place<<<nwin + 3, kDispWG, 0, st>>>(b.ids, T, K, E, nwin, b.masks, b.tiles, b.ntiles, b.perm, b.inv, sp);
   }
   {
     HookScope k(hook, "pf_gate_up", st);

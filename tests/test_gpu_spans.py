@@ -43,6 +43,29 @@ def test_spans(gt, dt, H, F):
     check(gt, dt, H, F, h.CODEBOOKS)
 
 
+@pytest.mark.parametrize("gt", [Q4, I3], ids=lambda v: moe.TYPE_NAMES[v])
+def test_span_lists(gt):
+    """The lists' order: an expert with more positions than the last class, several with as many spans as each other, rests of
+    one tile, experts without positions."""
+    counts = [80] * 9 + [1090, 0, 128, 128, 16, 1, 0, 65] + [144] * 4
+    E, T, H, F = len(counts), 1100, 512, 256
+    L = h.Layer(H, F, E, E, gt, Q8, has_shared=False, seed=77)
+    say("span lists", moe.TYPE_NAMES[gt])
+    blk = moe.MoeBlock(H, F, E, 15, gt, Q8, False, max_tokens=T)
+    r = np.random.default_rng(6)
+    x = h.tokens(78, T, H)
+    room = np.full(T, 16)  # jobs a token may still take
+    jobs = []
+    for e, c in enumerate(counts):
+        toks = r.permutation(np.flatnonzero(room))[:c]
+        room[toks] -= 1
+        jobs += [(L.experts[e], int(t), float(r.normal())) for t in toks]
+    y = blk.compute_many(jobs, x)
+    blk.close()
+    yo = h.orc_compute_many(gt, Q8, H, F, jobs, x)
+    assert np.array_equal(y, yo), h.max_abs(y, yo)
+
+
 def test_spans_swiglu_limit():
     check(XX, NL, 512, 256, h.CODEBOOKS, limit=0.05)
 
