@@ -919,6 +919,8 @@ __device__ __forceinline__ void unit_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
+// Where the activation buffers of a unit are restrict pointers, the function that takes them ends before the barrier: inside
+// it the compiler may take the barrier (and its memory clobber) for one that cannot touch them, and move their reads past it.
 
 // Q4_K, IQ3_S and Q8_0 on 16 x 16 int8 MFMA tiles (mfma_q4k.h, the decode path's tile; mfma_iq3s.h; mfma_q8_0.h):
 // wave w takes 16 weight rows (gate/up: matrix w / 2, rows 16 (w % 2) .. of the work-group's 32 of each; down: rows
@@ -1171,6 +1173,9 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
     }
     if constexpr (!kInPlace)
       if (more) raw = next;
+  };
+  const auto step = [&](uint32_t r, uint32_t u) {
+    body(r, u, abuf[u & 1], abuf[(u + 1) & 1]);
     __builtin_amdgcn_s_waitcnt(vm_wait(0));  // this wave's loads of unit u + 1 have landed ...
     // ... and every wave's, where this step loaded activations (so also every wave is done reading the buffer the
     // next step's loads refill), or, gate/up, before the up sums reuse the buffer. The other steps leave LDS as it
@@ -1181,7 +1186,7 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
 #pragma unroll 1
     for (uint32_t r = 0; r < R; r++) {
 #pragma unroll 1
-      for (uint32_t u = 0; u < U; u++) body(r, u, abuf[u & 1], abuf[(u + 1) & 1]);
+      for (uint32_t u = 0; u < U; u++) step(r, u);
       // Lane l holds rows row0 + r kRows + 4 (l / 16) + i of positions 16 pt + l % 16.
       const uint32_t l = lane_id(), r4 = 4 * (l / 16), c16 = l % 16;
 #pragma unroll
@@ -1195,7 +1200,7 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
     }
   } else {
 #pragma unroll 1
-    for (uint32_t u = 0; u < U; u++) body(0, u, abuf[u & 1], abuf[(u + 1) & 1]);
+    for (uint32_t u = 0; u < U; u++) step(0, u);
     // Lane l holds rows row0 + 4 (l / 16) + i of positions 16 pt + l % 16.
     const uint32_t l = lane_id(), r4 = 4 * (l / 16), c16 = l % 16;
 
@@ -1311,12 +1316,12 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
       };
       pass(rg, 0, accg);
       pass(ru, 1, accu);
-      if constexpr (next) {  // (after the last unit only the epilogue follows, which reads no activations)
-        __builtin_amdgcn_s_waitcnt(vm_wait(0));  // unit u + 1's loads (this wave's) ...
-        unit_barrier();                          // ... and every wave's; buffer u % 2 is free for unit u + 2
-      }
     };
     body(abuf[u & 1], abuf[(u + 1) & 1]);
+    if constexpr (decltype(kNext)::value) {  // (after the last unit only the epilogue follows, which reads no activations)
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));  // unit u + 1's loads (this wave's) ...
+      unit_barrier();                          // ... and every wave's; buffer u % 2 is free for unit u + 2
+    }
   };
 #pragma unroll 1
   for (uint32_t u = 0; u + 1 < U; u++) unit(u, std::true_type{});
@@ -1439,12 +1444,12 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
       };
       pass(rg, 0, accg);
       pass(ru, 1, accu);
-      if constexpr (next) {  // (after the last unit only the epilogue follows, which reads no activations)
-        __builtin_amdgcn_s_waitcnt(vm_wait(0));  // unit u + 1's loads (this wave's) ...
-        unit_barrier();                          // ... and every wave's; buffer u % 2 is free for unit u + 2
-      }
     };
     body(abuf[u & 1], abuf[(u + 1) & 1]);
+    if constexpr (decltype(kNext)::value) {  // (after the last unit only the epilogue follows, which reads no activations)
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));  // unit u + 1's loads (this wave's) ...
+      unit_barrier();                          // ... and every wave's; buffer u % 2 is free for unit u + 2
+    }
   };
 #pragma unroll 1
   for (uint32_t u = 0; u + 1 < U; u++) unit(u, std::true_type{});

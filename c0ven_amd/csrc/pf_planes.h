@@ -408,23 +408,30 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
       }
     }
   };
-  const auto unit = [&](uint32_t u, const uint8_t *__restrict__ buf, const float *__restrict__ ads, const uint8_t *__restrict__ sms,
-                        uint8_t *__restrict__ nbuf, float *__restrict__ nads, uint8_t *__restrict__ nsms) {
-    const uint32_t un = min(u + 1, U - 1);
+  // Two buffers, up to the wait: unit u's decode and gate products, and unit u + 1's activations on their way. buf (read)
+  // and nbuf (filled) are restrict pointers, so that the reads of buf do not wait for the loads into nbuf; the wait and the
+  // barrier are outside.
+  const auto gate_pass = [&](A &a, uint32_t un, const uint8_t *__restrict__ buf, const float *__restrict__ ads,
+                             const uint8_t *__restrict__ sms, uint8_t *__restrict__ nbuf, float *__restrict__ nads,
+                             uint8_t *__restrict__ nsms) {
+    dma(un, nbuf, nads, nsms);  // (every wave has passed the barrier after unit u - 1's products of that buffer)
+    pin_words(raw[0]);
+    raw[0].decode(a, lane_id(), grid);
+    pin_words(a);
+    raw[0].load(at(0), un, lane_id());
+    products(a, acc[0], buf, ads, sms);
+    pin_words(raw[1]);
+    raw[1].decode(a, lane_id(), grid);
+    pin_words(a);
+  };
+  const auto unit = [&](uint32_t u) {
+    const uint32_t un = min(u + 1, U - 1), b = u % kBufs, n = (u + 1) % kBufs;
     A a;
     if constexpr (kBufs == 2) {
-      dma(un, nbuf, nads, nsms);  // (every wave has passed the barrier after unit u - 1's products of that buffer)
-      pin_words(raw[0]);
-      raw[0].decode(a, lane_id(), grid);
-      pin_words(a);
-      raw[0].load(at(0), un, lane_id());
-      products(a, acc[0], buf, ads, sms);
-      pin_words(raw[1]);
-      raw[1].decode(a, lane_id(), grid);
-      pin_words(a);
+      gate_pass(a, un, abuf[b], adt[b], sums[b], abuf[n], adt[n], sums[n]);
       __builtin_amdgcn_s_waitcnt(vm_wait(0));  // this wave's loads of unit u + 1's activations (and gate's bytes) ...
       raw[1].load(at(1), un, lane_id());
-      products(a, acc[1], buf, ads, sms);
+      products(a, acc[1], abuf[b], adt[b], sums[b]);
       unit_barrier();  // ... and every wave's; buffer u % 2 is free
     } else {
       pin_words(raw[0]);
@@ -433,14 +440,14 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
       __builtin_amdgcn_s_waitcnt(vm_wait(0));  // unit u's activations (this wave's loads) ...
       unit_barrier();                          // ... and every wave's
       raw[0].load(at(0), un, lane_id());
-      products(a, acc[0], buf, ads, sms);
+      products(a, acc[0], abuf[0], adt[0], sums[0]);
       pin_words(raw[1]);
       raw[1].decode(a, lane_id(), grid);
       pin_words(a);
       raw[1].load(at(1), un, lane_id());
-      products(a, acc[1], buf, ads, sms);
+      products(a, acc[1], abuf[0], adt[0], sums[0]);
       unit_barrier();  // every wave is done with the buffer
-      if (u + 1 < U) dma(u + 1, nbuf, nads, nsms);
+      if (u + 1 < U) dma(u + 1, abuf[0], adt[0], sums[0]);
     }
   };
   dma(0, abuf[0], adt[0], sums[0]);
@@ -449,10 +456,7 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
     unit_barrier();
   }
 #pragma unroll 1
-  for (uint32_t u = 0; u < U; u++) {
-    const uint32_t b = u % kBufs, n = (u + 1) % kBufs;
-    unit(u, abuf[b], adt[b], sums[b], abuf[n], adt[n], sums[n]);
-  }
+  for (uint32_t u = 0; u < U; u++) unit(u);
   // Lane l holds rows 4 (l / 16) + i of positions 16 p + l % 16, gate and up alike.
   const uint32_t ln = lane_id(), l16 = ln & 15u, row0 = 64 * rb + 16 * wv + 4 * (ln >> 4);
 #pragma unroll
