@@ -30,7 +30,7 @@ typedef short s16x2_t __attribute__((ext_vector_type(2)));
 // the block's scale, in two planes of the x64 MFMA's order (step c: blocks 2 c, 2 c + 1), and the row's scale.
 struct PlaneA {
   v4i_t lo[4], hi[4];
-  float d;  // the A row's scale (times the type's factor, a power of two)
+  float d;  // the A row's scale
 };
 // Q4_K's: also the minima (f16, the x16 MFMA's operand) and their scale.
 struct PlaneAMin : PlaneA {
@@ -97,7 +97,7 @@ struct PlaneRaw<QT_IQ3_S> {
         a.hi[ib / 2][2 * (ib % 2) + j] = (int)((mul_bytes(gv, kh) ^ m) + x);
       }
     }
-    a.d = kFactor * h2f((uint16_t)dh);
+    a.d = h2f((uint16_t)dh);
   }
   static constexpr bool kNeg = true;
   static __device__ __forceinline__ int isum(int hi, int lo) { return __mul24(hi, -8) + lo; }
@@ -136,7 +136,7 @@ struct PlaneRaw<QT_IQ3_XXS> {
         a.lo[ib / 2][2 * (ib % 2) + j] = (int)((__builtin_amdgcn_perm(t.w, t.z, code) ^ m) + x);
       }
     }
-    a.d = kFactor * h2f((uint16_t)dh);
+    a.d = h2f((uint16_t)dh);
   }
   static constexpr bool kNeg = true;
   static __device__ __forceinline__ int isum(int hi, int lo) { return __mul24(hi, -64) + lo; }
@@ -178,7 +178,7 @@ struct PlaneRaw<QT_IQ2_S> {
         a.lo[ib / 2][2 * (ib % 2) + j] = (int)__builtin_amdgcn_perm(t.w, t.z, sel);
       }
     }
-    a.d = kFactor * h2f((uint16_t)dh);
+    a.d = h2f((uint16_t)dh);
   }
   static constexpr bool kNeg = true;
   static __device__ __forceinline__ int isum(int hi, int lo) { return __mul24(hi, -64) + lo; }
@@ -266,8 +266,8 @@ __device__ __forceinline__ void pin_words(T &r) {
   asm volatile("" ::: "memory");
 }
 
-// One position tile's: element i is row 4 (l / 16) + i, position l % 16 (d and a of lanes 0-15 used; the other three of the
-// instruction's products are 0 x 0, so zeros may lose their sign, which no sum they join can show).
+// One position tile's (scale_products): element i is row 4 (l / 16) + i, position l % 16 (d and a of lanes 0-15 used; the other
+// three of the instruction's products are 0 x 0).
 __device__ __forceinline__ v4f_t scale_products1(float d, float a, uint32_t lane) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(lane < 16 ? d : 0.0f, lane < 16 ? a : 0.0f, v4f_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
@@ -288,9 +288,11 @@ template <uint32_t kType>
 constexpr uint32_t plane_pos() { return kType == QT_Q4_K || kType == QT_IQ2_S ? 64u : 128u; }
 
 typedef float v16f_t __attribute__((ext_vector_type(16)));
-// d[16-row tile] x a[4 position tiles], each product rounded once (what __fmul_rn gives, subnormals and signed zeros
-// included: checked on 4 M random products): lane l's d is row l % 16's, its a position 16 (l / 16) + l % 16's; element
-// 4 b + i of the result is row 4 (l / 16) + i, position 16 b + l % 16. One matrix instruction for sixteen VALU ones.
+// d[16-row tile] x a[4 position tiles], each product rounded once, to a subnormal too, as __fmul_rn rounds it, but for the sign
+// of a zero: the instruction adds to +0, and -0 becomes +0. No output shows it: each product times an integer joins a sum that
+// starts from +0, and there either zero leaves the sum as it is. Lane l's d is row l % 16's, its a position
+// 16 (l / 16) + l % 16's; element 4 b + i of the result is row 4 (l / 16) + i, position 16 b + l % 16. One matrix
+// instruction for sixteen VALU ones.
 __device__ __forceinline__ v16f_t scale_products(float d, float a) {
   v16f_t z;
 #pragma unroll
@@ -401,7 +403,10 @@ __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3)))
         } else {
 #pragma unroll
           for (int i = 0; i < 4; i++) {
-            const float t = __fmul_rn(dd[4 * j + i], (float)Raw::isum(dh[i], dl[i]));
+            // The type's factor, a power of two, last, as UnitIQ3_XXS::term and UnitIQ2_S::term have it: in d it would take a
+            // product of the scales below 2^-126 and round it there. (Under 1% of a forward, the product being one more.)
+            float t = __fmul_rn(dd[4 * j + i], (float)Raw::isum(dh[i], dl[i]));
+            if constexpr (Raw::kFactor != 1.0f) t = __fmul_rn(Raw::kFactor, t);
             s[p][i] = Raw::kNeg ? __fsub_rn(s[p][i], t) : __fadd_rn(s[p][i], t);
           }
         }

@@ -16,7 +16,7 @@ Q8, Q4, I3, NL, XS, Q2, XX, S2 = (moe.QT_Q8_0, moe.QT_Q4_K, moe.QT_IQ3_S, moe.QT
                                   moe.QT_IQ3_XXS, moe.QT_IQ2_S)
 
 
-def check(gt, dt, H, F, codebooks, limit=0.0):
+def check(gt, dt, H, F, codebooks, limit=0.0, scales=None):
     E = len(COUNTS)
     L = h.Layer(H, F, E, E, gt, dt, has_shared=False, seed=910 + gt + F, swiglu_limit=limit)
     blk = moe.MoeBlock(H, F, E, E, gt, dt, False, max_tokens=260, swiglu_limit=limit)
@@ -25,6 +25,8 @@ def check(gt, dt, H, F, codebooks, limit=0.0):
     r = np.random.default_rng(5)
     x = h.tokens(911, 260, H)
     x[3] = 0.0  # a row whose scale is zero
+    if scales is not None:
+        x *= np.repeat(scales[r.integers(len(scales), size=(260, H // 256))], 256, axis=1).astype(np.float32)
     # Each expert's tokens in an order of its own; a token's jobs in expert order.
     toks = [set(r.permutation(260)[:c].tolist()) for c in COUNTS]
     jobs = [(L.experts[e], t, float(r.normal())) for t in range(260) for e in range(E) if t in toks[e]]
@@ -68,6 +70,14 @@ def test_span_lists(gt):
 
 def test_spans_swiglu_limit():
     check(XX, NL, 512, 256, h.CODEBOOKS, limit=0.05)
+
+
+@pytest.mark.parametrize("gt", [Q4, I3, XX, S2, XS], ids=lambda v: moe.TYPE_NAMES[v])
+def test_spans_tiny_scales(gt):
+    """Units whose activation scale makes its product with the weights' subnormal or zero beside units of ordinary size, and
+    rows of nothing else."""
+    say("spans, tiny scales", moe.TYPE_NAMES[gt])
+    check(gt, NL, 1024, 256, h.CODEBOOKS, scales=np.exp2([0.0, 0.0, -20.0, -85.0, -95.0, -105.0, -118.0]))
 
 
 @pytest.mark.parametrize("gt", [XX, S2], ids=lambda v: moe.TYPE_NAMES[v])
