@@ -205,8 +205,6 @@ struct moe_ctx {
   uint64_t ex_bytes = 0, ex_up = 0, ex_down = 0, sh_bytes = 0, sh_up = 0, sh_down = 0;
   uint32_t tmax = 0, tdec = 0, k1 = 0, gmax = 0;  // tokens a forward takes; of them, the decode kernel's
   PfBufs pf{};                                      // prefill scratch (max_tokens > tdec)
-  const int32_t *last_ids = nullptr;                // where the last forward left its ids and weights
-  const float *last_w = nullptr;
   uint32_t last_pf_T = 0;                           // tokens of the last prefill forward
   // Staging for the host-memory calls.
   float *x_dev = nullptr, *y_dev = nullptr, *w_stage = nullptr;
@@ -456,10 +454,20 @@ void launch(moe_ctx *c, const DecodeParams &p, hipStream_t s) {
   if (c->timing) timing_hook(c, "moe_decode", 1, s);
 }
 
-// The caller's ids and w (device memory, either may be null) are written by the kernels that select the top k, beside
-// the context's own (two copy launches after each forward took 4.5 us of a decode layer's 30 at one Q8_0 token); a
-// buffer off its 4-byte alignment, which only a copy takes, is copied to after the forward.
+// The caller's ids and w (device memory, either may be null) are written by the kernels that select the top k, the decode
+// kernel's in place of the context's own, the prefill kernels' beside them (two copy launches after each forward took
+// 4.5 us of a decode layer's 30 at one Q8_0 token); a buffer off its 4-byte alignment, which only a copy takes, is copied
+// to after the forward.
 bool words_aligned(const int32_t *ids, const float *w) { return (((uintptr_t)ids | (uintptr_t)w) & 3u) == 0; }
+
+// Where a forward of T tokens that the caller gave no buffers left its ids and weights.
+struct Routing {
+  const int32_t *ids;
+  const float *w;
+};
+Routing own_routing(const moe_ctx *c, uint32_t T) {
+  return T <= c->tdec ? Routing{c->ids, c->w} : Routing{c->pf.ids, c->pf.w};
+}
 
 void copy_routing(int32_t *ids, float *w, const int32_t *from_ids, const float *from_w, uint32_t n, hipStream_t s) {
   if (ids) check(hipMemcpyAsync(ids, from_ids, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s), "copy ids");
@@ -480,7 +488,6 @@ void forward_dev(moe_ctx *c, uint32_t layer, const float *x, uint32_t T, float *
     p.x = x, p.y = y;
     if (direct) p.ids = ids ? ids : p.ids, p.w = w ? w : p.w;
     launch(c, p, s);
-    c->last_ids = c->ids, c->last_w = c->w;
   } else {
     const moe_config &g = c->cfg;
     const Layer &L = c->layers[layer];
@@ -492,10 +499,10 @@ void forward_dev(moe_ctx *c, uint32_t layer, const float *x, uint32_t T, float *
                c->coded_ok ? c->coded : nullptr, L.rlsb, L.rmax, L.bias_max};
     PfHook hook{c->timing ? timing_hook : nullptr, c};
     check(prefill_forward(S, PL, c->pf, x, y, direct ? ids : nullptr, direct ? w : nullptr, s, hook), "prefill launch");
-    c->last_ids = c->pf.ids, c->last_w = c->pf.w, c->last_pf_T = T;
+    c->last_pf_T = T;
   }
   if (c->timing) c->ev_used++;
-  if (!direct) copy_routing(ids, w, c->last_ids, c->last_w, T * K, s);
+  if (!direct) copy_routing(ids, w, own_routing(c, T).ids, own_routing(c, T).w, T * K, s);
 }
 
 // Experts' bytes go up in the file's layout and are repacked on the device (moe_repack), at most kStageExperts at a time through
@@ -950,8 +957,8 @@ void forward_pinned(moe_ctx *c, uint32_t layer, const float *x, uint32_t T, uint
   check(hipGetLastError(), "upload x");
   forward_dev(c, layer, c->x_dev, T, c->y_dev, nullptr, nullptr, c->stream);
   hipLaunchKernelGGL(host_out, dim3((n16 + 2 * nr + 256) / 256), dim3(256), 0, c->stream, (uint4 *)yd, (const uint4 *)c->y_dev, n16,
-                     (uint32_t *)(yd + T * row), (const uint32_t *)c->err_flag, (const uint32_t *)c->last_ids,
-                     (const uint32_t *)c->last_w, nr);
+                     (uint32_t *)(yd + T * row), (const uint32_t *)c->err_flag, (const uint32_t *)own_routing(c, T).ids,
+                     (const uint32_t *)own_routing(c, T).w, nr);
   check(hipGetLastError(), "download y");
   check(hipStreamSynchronize(c->stream), "forward");
   for (uint32_t t = 0; t < T; t++) std::memcpy(y + t * y_stride, yh + t * row, row);
@@ -980,10 +987,10 @@ MOE_API moe_status moe_forward(moe_ctx *c, uint32_t layer, const float *x, uint3
                            hipMemcpyDeviceToHost, c->stream),
           "download y");
     if (route && route->ids)
-      check(hipMemcpyAsync(route->ids, c->last_ids, sizeof(int32_t) * ntok * K, hipMemcpyDeviceToHost, c->stream),
+      check(hipMemcpyAsync(route->ids, own_routing(c, ntok).ids, sizeof(int32_t) * ntok * K, hipMemcpyDeviceToHost, c->stream),
             "ids");
     if (route && route->w)
-      check(hipMemcpyAsync(route->w, c->last_w, sizeof(float) * ntok * K, hipMemcpyDeviceToHost, c->stream), "w");
+      check(hipMemcpyAsync(route->w, own_routing(c, ntok).w, sizeof(float) * ntok * K, hipMemcpyDeviceToHost, c->stream), "w");
     check(hipStreamSynchronize(c->stream), "forward");
     check_err(c);
   });
@@ -1081,7 +1088,6 @@ MOE_API moe_status moe_forward_hc_async(moe_ctx *c, uint32_t layer, float *R_dev
     const bool direct = words_aligned(ids_dev, w_dev);
     if (direct) p.ids = ids_dev ? ids_dev : p.ids, p.w = w_dev ? w_dev : p.w;
     launch(c, p, s);
-    c->last_ids = c->ids, c->last_w = c->w;
     if (c->timing) c->ev_used++;
     if (!direct) copy_routing(ids_dev, w_dev, c->ids, c->w, ntok * g.n_used, s);
   });
@@ -1103,10 +1109,10 @@ MOE_API moe_status moe_forward_hc(moe_ctx *c, uint32_t layer, float *R, uint32_t
                            c->stream),
             "download y");
     if (route && route->ids)
-      check(hipMemcpyAsync(route->ids, c->last_ids, sizeof(int32_t) * ntok * K, hipMemcpyDeviceToHost, c->stream),
+      check(hipMemcpyAsync(route->ids, own_routing(c, ntok).ids, sizeof(int32_t) * ntok * K, hipMemcpyDeviceToHost, c->stream),
             "ids");
     if (route && route->w)
-      check(hipMemcpyAsync(route->w, c->last_w, sizeof(float) * ntok * K, hipMemcpyDeviceToHost, c->stream), "w");
+      check(hipMemcpyAsync(route->w, own_routing(c, ntok).w, sizeof(float) * ntok * K, hipMemcpyDeviceToHost, c->stream), "w");
     check(hipStreamSynchronize(c->stream), "forward_hc");
     check_err(c);
   });
@@ -1280,7 +1286,7 @@ MOE_API moe_status moe_compute_many(moe_ctx *c, const moe_cm_job *jobs, uint32_t
                  c->coded_ok ? c->coded : nullptr, nullptr, 0.0f, 0.0f};
       PfHook hook{c->timing ? timing_hook : nullptr, c};
       check(prefill_jobs(S, PL, c->pf, c->x_dev, c->y_dev, s, hook), "prefill launch");
-      c->last_ids = c->pf.ids, c->last_w = c->pf.w, c->last_pf_T = ntok;
+      c->last_pf_T = ntok;
       check(hipStreamSynchronize(s), "pre-routed prefill");  // the host's ids and w must outlive the copies
     }
     check(hipMemcpy2DAsync(y, y_stride * sizeof(float), c->y_dev, H * sizeof(float), H * sizeof(float), ntok,

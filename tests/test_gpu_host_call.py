@@ -33,3 +33,24 @@ def test_host_call_rows(T):
         assert (yb[:, H:] == 7.0).all()
         assert not route or (np.array_equal(ids, io) and np.array_equal(w, wo))
     blk.close()
+
+
+@pytest.mark.parametrize("T", [3, 18])
+def test_host_call_after_device_calls(T):
+    """The routing of a host call is its own forward's, whatever buffers the forwards before it wrote theirs to."""
+    say("host call after device calls", T)
+    H, K = 512, 4
+    L = h.Layer(H, 256, 32, K, moe.QT_Q4_K, moe.QT_Q8_0, seed=83, zipf=1.1)
+    blk = L.block(max_tokens=20, exact_router=True)
+    L.upload(blk)
+    d = h.Dev()
+    ids, w, y = d.alloc(20 * K * 4), d.alloc(20 * K * 4), d.alloc(20 * H * 4)
+    for i, (a, b) in enumerate(((ids, w), (None, w), (ids, None))):
+        for n in (2, 19):
+            blk.forward_async(0, d.put(h.tokens(90 + i, n, H)), n, y, a, b)
+        x = h.tokens(84 + i, T, H)
+        yo, io, wo = L.oracle_forward(x)
+        y2, i2, w2 = blk.forward(0, x)
+        assert np.array_equal(y2, yo) and np.array_equal(i2, io) and np.array_equal(w2, wo)
+    d.free()
+    blk.close()
