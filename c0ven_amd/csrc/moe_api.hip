@@ -518,7 +518,8 @@ uint64_t stage_bytes(const RepackShape &s) {
   return n;
 }
 
-// The staging buffer, for n (at most kStageExperts) experts of the context's largest file layout.
+// The staging buffer, for n (at most kStageExperts) experts of the context's largest file layout. moe_open makes it for one,
+// so that a load allocates nothing; where there is no room for more, it stays as it is and takes an expert at a time.
 void stage_experts(moe_ctx *c, uint32_t n) {
   if (n <= c->stage_slots) return;
   check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
@@ -528,15 +529,21 @@ void stage_experts(moe_ctx *c, uint32_t n) {
   };
   c->stage_stride = std::max(bytes(g.gate_type, g.gate_type, g.down_type),
                              g.has_shared ? bytes(g.sh_gate_type, g.sh_up_type, g.sh_down_type) : uint64_t(0));
+  const uint64_t slot = c->stage_stride + sizeof(RepackExpert);
   void *p = nullptr;
-  check(hipMalloc(&p, n * (c->stage_stride + sizeof(RepackExpert))), "hipMalloc");
+  const hipError_t e = hipMalloc(&p, n * slot);
+  if (e != hipSuccess && c->stage) {
+    (void)hipGetLastError();
+    return;
+  }
+  check(e, "hipMalloc");
   if (c->stage) {
     c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void *)c->stage));
-    c->dev_bytes -= c->stage_slots * (c->stage_stride + sizeof(RepackExpert));
+    c->dev_bytes -= c->stage_slots * slot;
     (void)hipFree(c->stage);
   }
   c->allocs.push_back(p);
-  c->stage = (uint8_t *)p, c->stage_slots = n, c->dev_bytes += n * (c->stage_stride + sizeof(RepackExpert));
+  c->stage = (uint8_t *)p, c->stage_slots = n, c->dev_bytes += n * slot;
 }
 
 // Experts ew[0 .. n - 1] (n at most the staging buffer's) into the device layout at dst[i], on a stream, and waits for it.
@@ -686,6 +693,7 @@ MOE_API moe_status moe_open(const moe_config *cfg, moe_ctx **out) {
       check(hipHostGetDevicePointer(&d, h, 0), "hipHostGetDevicePointer");
       c->io_dev = (uint8_t *)d;
     }
+    stage_experts(c, 1);
     c->ids_stage = c->alloc<int32_t>((uint64_t)T * K1);
     c->w_stage = c->alloc<float>((uint64_t)T * K1);
     if (TM > T) {  // the prefill path's scratch (a pre-routed call's token may take n_used + 1 jobs)
@@ -898,7 +906,6 @@ MOE_API moe_status moe_load_expert(moe_ctx *c, uint32_t layer, uint32_t expert, 
     const uint64_t gb = matrix_bytes(gt, g.n_ff, g.n_embd), ub = matrix_bytes(ut, g.n_ff, g.n_embd);
     uint8_t *dst = shared ? c->layers[layer].shared : c->layers[layer].experts + (uint64_t)expert * c->ex_bytes;
     const RepackShape sh{{gt, ut, dt}, {g.n_ff, g.n_ff, g.n_embd}, {g.n_embd, g.n_embd, g.n_ff}, {0, gb, gb + ub}};
-    stage_experts(c, 1);
     const moe_expert_weights ew{gate, up, down, 1, {0, 0}};
     // The null stream, as any load: it waits for the work of the blocking streams that may read the old weights.
     repack_staged(c, sh, &ew, &dst, 1, nullptr);

@@ -38,3 +38,14 @@ def test_repack_of_borrowed_experts(types, n):
     yo = h.orc_compute_many(gt, dt, H, F, ojobs, x)
     assert np.array_equal(y, yo), h.max_abs(y, yo)
     blk.close()
+
+
+def test_load_allocates_nothing():
+    """A context holds all that its loads need once it is open."""
+    say("loads allocate nothing")
+    L = h.Layer(512, 256, 8, 2, moe.QT_Q4_K, moe.QT_Q8_0, moe.QT_Q8_0, moe.QT_Q8_0, seed=3)
+    blk = L.block()
+    held = blk.device_bytes()
+    L.upload(blk)
+    assert blk.device_bytes() == held
+    blk.close()
