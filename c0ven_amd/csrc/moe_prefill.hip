@@ -1629,7 +1629,7 @@ void launch_planes(uint32_t type, uint32_t U, uint32_t ns, uint32_t F, const PfG
 }
 
 // Routed down of the q8_0 family on pf_down_q8 (spans of kDownPos positions), H rows of F values.
-constexpr bool down_q8(uint32_t type, uint32_t F) { return q8_family(type) && down_lds(F) <= kDownMaxLds; }
+constexpr bool down_q8(uint32_t type, uint32_t F) { return q8_family(type) && down_lds(F) + kDownStatic <= kDownMaxLds; }
 void launch_down_q8(uint32_t type, uint32_t F, uint32_t ns, uint32_t H, const PfGemm &g, hipStream_t s) {
   PfGemm q = g;
   q.U = units_of(F), q.K = F, q.row_blocks = H / 64;

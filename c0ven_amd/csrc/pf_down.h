@@ -88,9 +88,12 @@ constexpr uint32_t kDownPos = 64;  // positions a work-group takes
 constexpr uint32_t down_lds(uint32_t F) {
   return kDownPos * (F / 256 * 256 + (F % 256 == 0 ? 0 : F % 256 == 128 ? 128 : 256) + (F + 255) / 256 * 32);
 }
-constexpr uint32_t kDownMaxLds = 64 * 1024;  // two work-groups a CU at the most; larger F keep pf_gemm16
+constexpr uint32_t kDownStatic = 4 * kDownPos;  // the positions' offsets, beside them
+// The most a work-group takes, so that two fit a CU: F to 896 (Q8_0 2048 x 896: 5% of a forward less than with pf_gemm16 at
+// 2048 tokens); larger F, which were not measured, keep pf_gemm16.
+constexpr uint32_t kDownMaxLds = 65 * 1024;
 // 64-row groups a work-group walks: fewer where the launch would have less than two rounds of the device's work-groups (three a
-// CU). nrb (n_embd / 64) is a multiple of 8.
+// CU to F 640, two above). nrb (n_embd / 64) is a multiple of 8.
 constexpr uint32_t kDownGroups = 1536;
 __host__ __device__ constexpr uint32_t down_walk(uint32_t nspans, uint32_t nrb) {
   uint32_t W = 8;
@@ -101,7 +104,7 @@ __host__ __device__ constexpr uint32_t down_walk(uint32_t nspans, uint32_t nrb) 
 template <uint32_t kType>
 __global__ void __launch_bounds__(kPfWG) __attribute__((amdgpu_waves_per_eu(3))) pf_down_q8(PfGemm g) {
   extern __shared__ __align__(16) uint8_t lds[];
-  __shared__ uint32_t arow[kDownPos];
+  __shared__ uint32_t arow[kDownStatic / 4];
   const uint32_t U = g.U, nsp = *g.nspans, W = down_walk(nsp, g.row_blocks);
   uint32_t sp, rb;
   if (!span_item(blockIdx.x, g.row_blocks / W, nsp, &sp, &rb)) return;

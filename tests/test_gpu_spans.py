@@ -38,7 +38,8 @@ def check(gt, dt, H, F, codebooks, limit=0.0, scales=None):
 
 @pytest.mark.parametrize("gt,dt,H,F", [(Q4, NL, 512, 640), (I3, Q2, 512, 320), (XX, NL, 1024, 640), (S2, Q8, 512, 256),
                                        (XS, NL, 512, 448), (I3, Q4, 2560, 512), (S2, Q2, 2560, 640), (Q8, Q8, 512, 512),
-                                       (Q4, Q8, 512, 960)],
+                                       (Q4, Q8, 512, 960), (Q4, Q8, 512, 896), (XX, NL, 512, 896), (I3, NL, 512, 768),
+                                       (S2, Q2, 512, 704)],
                          ids=lambda v: moe.TYPE_NAMES.get(v, str(v)))
 def test_spans(gt, dt, H, F):
     say("spans", (moe.TYPE_NAMES[gt], moe.TYPE_NAMES[dt], H, F))
@@ -65,6 +66,38 @@ def test_span_lists(gt):
     y = blk.compute_many(jobs, x)
     blk.close()
     yo = h.orc_compute_many(gt, Q8, H, F, jobs, x)
+    assert np.array_equal(y, yo), h.max_abs(y, yo)
+
+
+@pytest.mark.parametrize("spans,walk", [(80, 2), (160, 4), (320, 8)])
+@pytest.mark.parametrize("dt", [Q8, NL, Q2], ids=lambda v: moe.TYPE_NAMES[v])
+def test_down_walk(dt, spans, walk):
+    """A work-group of the q8_0 family's down that walks several 64-row groups (their number follows from the spans and n_embd:
+    pf_down.h's down_walk, restated), rows that end in half a unit, spans of one position, of several tiles and full ones."""
+    H, F, E, K = 2560, 640, spans - 4, 15
+    groups = lambda w: (spans + 7) // 8 * 8 * (H // 64 // w)  # noqa: E731
+    assert next(w for w in (8, 4, 2, 1) if w == 1 or groups(w) >= 1536) == walk
+    counts = [1] * (E - 12) + [16, 17, 33, 48, 63, 64, 64, 50, 128, 100, 65, 70]
+    assert sum((c + 63) // 64 for c in counts) == spans
+    say("down walk", (moe.TYPE_NAMES[dt], spans, walk))
+    L = h.Layer(H, F, 4, 1, Q4, dt, has_shared=False, seed=55)
+    T = 130
+    blk = moe.MoeBlock(H, F, 64, K, Q4, dt, False, max_tokens=T)
+    r = np.random.default_rng(spans)
+    x = h.tokens(56, T, H)
+    room = np.full(T, K + 1)
+    jobs, ojobs = [], []
+    for e, c in enumerate(counts):
+        g, u, d = L.experts[e % 4]
+        mine = (g.copy(), u, d)  # an expert of its own by its gate's address
+        toks = np.argsort(-room + 0.5 * r.random(T))[:c]
+        room[toks] -= 1
+        for t in toks:
+            w = float(r.normal())
+            jobs.append((mine, int(t), w)), ojobs.append((L.experts[e % 4], int(t), w))
+    y = blk.compute_many(jobs, x)
+    blk.close()
+    yo = h.orc_compute_many(Q4, dt, H, F, ojobs, x)
     assert np.array_equal(y, yo), h.max_abs(y, yo)
 
 
