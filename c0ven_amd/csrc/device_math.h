@@ -116,20 +116,13 @@ constexpr int kDppShr1 = 0x111;  // row_shr:1 (lane - 1 within a row of 16)
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
 
-// The wave's largest / smallest u32, wave-uniform.
+// The wave's largest u32, wave-uniform.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   v = max(v, dpp_u32<kDppXor1>(v));
   v = max(v, dpp_u32<kDppXor2>(v));
   v = max(v, dpp_u32<kDppHalfMirror>(v));
   v = max(v, dpp_u32<kDppMirror>(v));
   return max(max(readlane_u32(v, 0), readlane_u32(v, 16)), max(readlane_u32(v, 32), readlane_u32(v, 48)));
-}
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-  v = min(v, dpp_u32<kDppXor1>(v));
-  v = min(v, dpp_u32<kDppXor2>(v));
-  v = min(v, dpp_u32<kDppHalfMirror>(v));
-  v = min(v, dpp_u32<kDppMirror>(v));
-  return min(min(readlane_u32(v, 0), readlane_u32(v, 16)), min(readlane_u32(v, 32), readlane_u32(v, 48)));
 }
 
 template <int kCtrl>

@@ -1233,9 +1233,9 @@ __device__ __forceinline__ void pin(Iq3sRaw &r) {
                "+v"(r.dh[0]), "+v"(r.dh[1]), "+v"(r.dh[2]), "+v"(r.dh[3]) :: "memory");
 }
 
-// Q4_K gate/up at three waves a SIMD: a unit's gate products come before its up products, so that one matrix's
-// decoded operands are live at a time (150 registers; the activation operands are read from LDS once for each), and
-// the activations are loaded one unit ahead into two LDS buffers (44 KB a work-group, three a CU). Wave w takes rows
+// The shared expert's Q4_K gate/up (tokens in order) at three waves a SIMD: a unit's gate products come before its up
+// products, so that one matrix's decoded operands are live at a time (150 registers; the activation operands are read
+// from LDS once for each), and the activations are loaded one unit ahead into two LDS buffers (44 KB a work-group, three a CU). Wave w takes rows
 // 16 w .. 16 w + 15 of gate and of up (a work-group 64 rows of each, kPos = 64 positions, four waves), so SwiGLU pairs
 // gate and up in the same lane. A matrix's weights are decoded, then the registers of its raw bytes take the next
 // unit's loads (buffer loads on scalar bases), which the end of the unit waits for with the activations; the
@@ -1250,27 +1250,16 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
   __shared__ uint32_t arow_lds[kPos];
   __shared__ uint64_t tab[32];
   const uint32_t nrb = g.row_blocks;
-  const uint32_t nch = g.shared_T ? (g.shared_T + kPos - 1) / kPos : *g.ntiles, n = nch * nrb;
+  const uint32_t nch = (g.shared_T + kPos - 1) / kPos, n = nch * nrb;
   if (blockIdx.x >= n) return;
   const uint32_t L = xcd_logical(blockIdx.x, n);
-  const uint32_t ch_i = L / nrb, rb = L % nrb;
-  uint32_t start, count, e;
-  if (g.shared_T) {
-    start = kPos * ch_i;
-    count = min(kPos, g.shared_T - start), e = 0;
-  } else {
-    const MoeTile tl = g.tiles[ch_i];
-    start = tl.start, count = tl.count, e = tl.slot;
-  }
+  const uint32_t rb = L % nrb, start = kPos * (L / nrb), count = min(kPos, g.shared_T - start);
   const uint32_t tid = tid_fresh();
   if (tid < 32) tab[tid] = kExp2Tab[tid];
-  if (tid < kPos) {
-    const uint32_t pos = start + tid;
-    arow_lds[tid] = tid < count ? (g.perm ? g.perm[pos] / g.K : pos) : 0xffffffffu;
-  }
+  if (tid < kPos) arow_lds[tid] = tid < count ? start + tid : 0xffffffffu;
   __syncthreads();
   const uint32_t row0 = rb * kRows + 16 * (uint32_t)__builtin_amdgcn_readfirstlane(wave_id()), lane = lane_id();
-  const uint8_t *Mg = g.mat + (uint64_t)e * g.stride, *Mu = Mg + g.up_off;
+  const uint8_t *Mg = g.mat, *Mu = Mg + g.up_off;
   const uint32_t npt = (count + 15) / 16;  // 16-position tiles with positions
   Dma<kPos, kWaves> dma;
   dma.plan(arow_lds, U);
@@ -1337,14 +1326,15 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
     }
 }
 
-// IQ3_S gate/up at three waves a SIMD, in pf_gate_up_q4k's form: gate's products before up's, the activations one
-// unit ahead in two LDS buffers, plain barriers. A block's A operand is decoded from the raw words (grid lookups in
-// LDS) just before its MFMAs, so only the raw words and one block's operand are live (144 registers); each block's
-// dots times the row's odd block scale are added to the unit's integer sums in block order, then d ad isum as
+// The shared expert's IQ3_S gate/up at three waves a SIMD, in pf_gate_up_q4k's form: gate's products before up's, the
+// activations one unit ahead in two LDS buffers, plain barriers. A block's A operand is decoded from the raw words (grid
+// lookups in LDS) just before its MFMAs, so only the raw words and one block's operand are live (144 registers); each
+// block's dots times the row's odd block scale are added to the unit's integer sums in block order, then d ad isum as
 // UnitIQ3_S::term, units added in sequence. The raw registers take the next unit's loads (buffer loads on scalar
 // bases, Iq3sBuf) once the pass has read them. Against the earlier form (both matrices in one wave, 220 registers,
-// two waves a SIMD, activations two units ahead): 367 -> 350 us a launch at config 5p; the buffer loads (in place
-// of global loads, 168 registers and a reload from scratch a unit) 358 -> 329 us.
+// two waves a SIMD, activations two units ahead) a launch over config 5p's routed experts, which it then ran too, took
+// 350 us instead of 367; with buffer loads (in place of global loads, 168 registers and a reload from scratch a unit)
+// 329 instead of 358.
 template <uint32_t kPos>
 __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3))) pf_gate_up_iq3s(PfGemm g) {
   const uint32_t U = g.U;
@@ -1355,28 +1345,17 @@ __global__ void __launch_bounds__(4 * kPos) __attribute__((amdgpu_waves_per_eu(3
   __shared__ uint64_t tab[32];
   __shared__ uint32_t grid_lds[512];
   const uint32_t nrb = g.row_blocks;
-  const uint32_t nch = g.shared_T ? (g.shared_T + kPos - 1) / kPos : *g.ntiles, n = nch * nrb;
+  const uint32_t nch = (g.shared_T + kPos - 1) / kPos, n = nch * nrb;
   if (blockIdx.x >= n) return;
   const uint32_t L = xcd_logical(blockIdx.x, n);
-  const uint32_t ch_i = L / nrb, rb = L % nrb;
-  uint32_t start, count, e;
-  if (g.shared_T) {
-    start = kPos * ch_i;
-    count = min(kPos, g.shared_T - start), e = 0;
-  } else {
-    const MoeTile tl = g.tiles[ch_i];
-    start = tl.start, count = tl.count, e = tl.slot;
-  }
+  const uint32_t rb = L % nrb, start = kPos * (L / nrb), count = min(kPos, g.shared_T - start);
   const uint32_t tid = tid_fresh();
   if (tid < 32) tab[tid] = kExp2Tab[tid];
   for (uint32_t i = tid; i < 512; i += 64 * kWaves) grid_lds[i] = kIq3sGridPf[i];
-  if (tid < kPos) {
-    const uint32_t pos = start + tid;
-    arow_lds[tid] = tid < count ? (g.perm ? g.perm[pos] / g.K : pos) : 0xffffffffu;
-  }
+  if (tid < kPos) arow_lds[tid] = tid < count ? start + tid : 0xffffffffu;
   __syncthreads();
   const uint32_t row0 = rb * kRows + 16 * (uint32_t)__builtin_amdgcn_readfirstlane(wave_id()), lane = lane_id();
-  const uint8_t *Mg = g.mat + (uint64_t)e * g.stride, *Mu = Mg + g.up_off;
+  const uint8_t *Mg = g.mat, *Mu = Mg + g.up_off;
   const uint32_t npt = (count + 15) / 16;  // 16-position tiles with positions
   Dma<kPos, kWaves> dma;
   dma.plan(arow_lds, U);
@@ -1488,8 +1467,8 @@ namespace {
 
 // Positions a gate/up work-group takes for a weight type (the kernel's kPos).
 constexpr uint32_t gu_pos(uint32_t) { return MOE_TILE; }
-// The gate/up types that run on pf_gate_up_q4k / pf_gate_up_iq3s (gate and up of a row in one wave); the others on
-// pf_gemm16.
+// The shared expert's gate/up types that run on pf_gate_up_q4k / pf_gate_up_iq3s (gate and up of a row in one wave); the others,
+// and the routed experts' types without planes (plane_len), on pf_gemm16.
 constexpr bool gu_fused(uint32_t type) { return type == QT_Q4_K || type == QT_IQ3_S; }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1655,9 +1634,10 @@ struct HookScope {
   }
 };
 
-// Gate/up (SwiGLU into h) over nx tiles or chunks (at most; the kernel reads how many there are): Q4_K and IQ3_S on
-// pf_gate_up_q4k / pf_gate_up_iq3s (gu_pos positions and rows of each a work-group), the other types on pf_gemm16
-// (64-position tiles, 32 rows of gate and of up a work-group).
+// Gate/up (SwiGLU into h) over nx chunks of the shared expert's tokens, or nx tiles at most of the routed experts' (the kernel reads
+// how many there are): the shared Q4_K and IQ3_S on pf_gate_up_q4k / pf_gate_up_iq3s (gu_pos positions and rows of each a
+// work-group; the routed ones run on the planes), the other types on pf_gemm16 (64-position tiles, 32 rows of gate and of up
+// a work-group).
 // Explicit instantiations: with only the implicit ones, this compiler's host pass emits the launch stub of the
 // first instantiation of a kernel template whose body holds a lambda and silently drops the later ones (and with
 // them launch_gemm<false>), which then fail at load time as undefined symbols.
