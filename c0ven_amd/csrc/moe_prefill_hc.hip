@@ -188,10 +188,37 @@ __global__ void __launch_bounds__(kHcWG) pf_hc_digits(const uint16_t *A0, uint32
 struct Side {
   double norm, units, lost, top;
 };
+// What side_of reads of n consecutive rows or tokens from i on, all in flight together (left to the compiler, a side's lsb is
+// read only once its lost bits are known to be none, and each side is waited for before the next one's loads: the up
+// product 69 us instead of 61 at 1000 tokens of H 2560, lr 320). n 4: i a multiple of 4, the arrays 16-byte aligned.
+template <uint32_t n>
+struct SideRaw {
+  uint32_t norm[n][2], lsb[n], exp[n], lost[n];
+  __device__ __forceinline__ void load(const double *nm, const int *l, const HcGrid &g, uint32_t i) {
+    if constexpr (n == 4) {
+      *(uint4 *)&norm[0] = *(const uint4 *)(nm + i), *(uint4 *)&norm[2] = *(const uint4 *)(nm + i + 2);
+      *(uint4 *)lsb = *(const uint4 *)(l + i), *(uint4 *)exp = *(const uint4 *)(g.exp + i), *(uint4 *)lost = *(const uint4 *)(g.lost + i);
+    } else {
+      *(uint2 *)&norm[0] = *(const uint2 *)(nm + i), lsb[0] = l[i], exp[0] = g.exp[i], lost[0] = g.lost[i];
+    }
+  }
+  __device__ __forceinline__ void arrived() {
+#pragma unroll
+    for (uint32_t k = 0; k < n; k++)
+      asm volatile("" : "+v"(norm[k][0]), "+v"(norm[k][1]), "+v"(lsb[k]), "+v"(exp[k]), "+v"(lost[k]));
+  }
+  __device__ __forceinline__ Side side(uint32_t k, bool wide) const {
+    const uint32_t m = wide ? 0u : lost[k];
+    const int e = max((int)exp[k], 1);
+    const double r = __hiloint2double((int)norm[k][1], (int)norm[k][0]);
+    return {r, m ? __builtin_inf() : ldexp(r, -(int)lsb[k]), ldexp((double)m, e - 172), ldexp(1.0, e - 126)};
+  }
+};
 __device__ __forceinline__ Side side_of(const double *norm, const int *lsb, const HcGrid &g, uint32_t i, bool wide) {
-  const uint32_t n = wide ? 0u : g.lost[i];
-  const int e = max(g.exp[i], 1);
-  return {norm[i], n ? __builtin_inf() : ldexp(norm[i], -lsb[i]), ldexp((double)n, e - 172), ldexp(1.0, e - 126)};
+  SideRaw<1> r;
+  r.load(norm, lsb, g, i);
+  r.arrived();
+  return r.side(0, wide);
 }
 
 // Whether the sum v of a row's and a token's bf16 products rounds to fp32 as the fixed order's does. Exact: no bits lost,
@@ -414,7 +441,8 @@ __device__ __forceinline__ void digit_products(const uint8_t *A, uint32_t M, con
 // kUp: one part; the sums are certified here (rows' and tokens' sides) and written as fp32 to out32 (N x M), an open one's
 // (token, row) to the list open (pf_hc_up_fix writes it). Otherwise the part's fp64 sums go to part (nsplit x N x M), and
 // whether a 32 x 32 tile was wide to wide_map (token tiles x row tiles).
-// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 46 us (51 with the lowest digits always loaded) and up 59, where the fp64 matrix cores took 162 and 141.
+// T 1000, H 2560, lr 320 (2 x 3.3 G products): down 49 us (5 more with the lowest digits always loaded) and up 61, where the
+// fp64 matrix cores took 162 and 141.
 template <bool kUp>
 __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_t M, const uint8_t *B, uint32_t N,
                                                        const uint16_t *A0, uint32_t M0, const uint16_t *A1,
@@ -425,7 +453,7 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
                                                        uint32_t *open, uint32_t *cnt) {
   const uint32_t nmt = (M + 63) / 64, split = blockIdx.x % nsplit, item = blockIdx.x / nsplit;
   const uint32_t mt = item % nmt, nt = item / nmt, cs = nch / nsplit;
-  const uint32_t lane = lane_of(), w = threadIdx.x >> 6, g = lane / 16, c16 = lane % 16;
+  const uint32_t lane = lane_of(), w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane / 16, c16 = lane % 16;
   const uint32_t m0 = 64 * mt + 32 * (w & 1), n0 = 64 * nt + 32 * (w >> 1);
   // 16 x 16 tiles wholly past the rows or the tokens are skipped: a wave with none returns (the kernel has no barrier),
   // the others repeat their first tile's operands and drop its sums.
@@ -439,6 +467,15 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
     wide_products(A0, M0, A1, M, Bb, N, K, 64 * split * cs, min(K, 64 * (split + 1) * cs), m0, n0, v);
   else
     digit_products(A, M, B, N, nch, split, cs, m0, n0, i1, j1, gr, gt, v);
+  SideRaw<4> rr[2];
+  SideRaw<1> tr[2];
+  if constexpr (kUp) {
+#pragma unroll
+    for (uint32_t f = 0; f < 2; f++)
+      rr[f].load(rn, rl, gr, min(m0 + 16 * f + 4 * g, M - 4)), tr[f].load(tn, tl, gt, min(n0 + 16 * f + c16, N - 1));
+#pragma unroll
+    for (uint32_t f = 0; f < 2; f++) rr[f].arrived(), tr[f].arrived();
+  }
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const uint32_t row = m0 + 16 * i + 4 * g;
@@ -446,13 +483,13 @@ __global__ void __launch_bounds__(kHcWG, 2) pf_hc_gemm(const uint8_t *A, uint32_
     Side rs[4];
     if constexpr (kUp)
 #pragma unroll
-      for (int q = 0; q < 4; q++) rs[q] = side_of(rn, rl, gr, row + q, wide);
+      for (int q = 0; q < 4; q++) rs[q] = rr[i].side(q, wide);
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       const uint32_t tok = n0 + 16 * j + c16;
       if (tok >= N) continue;
       if constexpr (kUp) {
-        const Side ts = side_of(tn, tl, gt, tok, wide);
+        const Side ts = tr[j].side(0, wide);
         *(float4 *)(out32 + (uint64_t)tok * M + row) =
             make_float4((float)v[i][j][0], (float)v[i][j][1], (float)v[i][j][2], (float)v[i][j][3]);
 #pragma unroll
