@@ -45,12 +45,12 @@ CONFIGS = {
     "hc2": dict(name="config2 + hyper-connection mix and combine (hc_lr 256): verify T=8, Q4_K, Zipf(1.1)",
                 types=(12, 12, 12, 12), T=8, zipf=1.1, hc_lr=256),
 }
-FP64_PEAK_TFLOPS = 78.6  # dense fp64 MFMA, MI355X
 H, F, E, K = 2048, 512, 512, 10
 HBM_PEAK_GBS = 8000.0
 INT8_PEAK_TOPS = 5000.0  # dense int8 MFMA, MI355X
-# The routed gate/up kernel of a gate type (the launch the prefill roofline is quoted on); pf_gemm16 for the others.
-GU_KERNEL = {12: "pf_gate_up_q4k", 21: "pf_gate_up_iq3s"}  # Q4_K, IQ3_S
+# The routed gate/up kernel of a gate type (the launch the prefill roofline is quoted on): Q4_K, IQ3_XXS, IQ3_S, IQ2_S and
+# IQ4_XS; pf_gemm16 for the others.
+GU_KERNEL = dict.fromkeys((12, 18, 21, 22, 23), "pf_gate_up_planes")
 
 
 class Hip:
@@ -402,10 +402,11 @@ def hc(args, cfg, moe, h):
     D = 4 * H
     flop = 2.0 * T * (lr + 4) * D + 2.0 * T * D * lr
     mix_ms = hc_ms - plain_ms
-    if T > 16:  # the prefill kernels: fp64 matrix cores
+    if T > 16:  # the prefill kernels: nine int8 digit products a product (sixteen where a lowest digit is not zero)
+        peak = INT8_PEAK_TOPS / 9
         roof = {"bound": "mfma", "kernel": "pf_hc_gemm (down and up) and the mix's other kernels",
-                "achieved": round(flop / (mix_ms * 1e-3) / 1e12, 2), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(flop / (mix_ms * 1e-3) / 1e12 / FP64_PEAK_TFLOPS, 4), "traffic": None,
+                "achieved": round(flop / (mix_ms * 1e-3) / 1e12, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+                "frac": round(flop / (mix_ms * 1e-3) / 1e12 / peak, 4), "traffic": None,
                 "algorithmic_flop_per_launch": flop, "avg_launch_ms": round(mix_ms, 4)}
     else:  # the decode launch's items: the module's weights read once (bf16 W_down, W_inject, W_up)
         wbytes = 2.0 * ((lr + 4) * D + D * lr)

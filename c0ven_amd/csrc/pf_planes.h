@@ -10,7 +10,7 @@
 // are live at a time (three waves a SIMD).
 // Measured against the block-by-block kernels at their 64-position tiles (one launch, top 10 of 512 experts, Zipf): IQ2_S
 // 2560 x 640 at 4096 tokens 1331 -> 502 us, IQ3_XXS at 301 tokens 183 -> 106, IQ3_S 2048 x 512 at 2048 tokens 320 -> 209,
-// Q4_K 178 -> 166 and at 37 tokens 81 -> 74. An earlier form that decoded into LDS for 256 positions and took the activations
+// Q4_K 178 -> 166 and at 37 tokens 81 -> 74; a whole forward of IQ4_XS 2048 x 512 at 2048 tokens 748 -> 500. An earlier form that decoded into LDS for 256 positions and took the activations
 // straight into registers measured 717, 150, 277 and 309 us: its activation reads were what bounded it.
 #pragma once
 
@@ -281,9 +281,15 @@ __device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, void *lds, u
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 4, voff, soff, 0, 0);
 }
 
-// Positions a work-group takes (its spans; both lengths measured: Q4_K at 2048 tokens 64 166, 128 170 us, at 37 tokens 74, 85). Where decoding a unit is cheap beside its products (Q4_K: 100 VALU instructions a
+// Positions a work-group takes (its spans). Where decoding a unit is cheap beside its products (Q4_K: 100 VALU instructions a
 // matrix; IQ2_S), 64 in two activation buffers; where it is dear (IQ3_S, IQ3_XXS, IQ4_XS: 230-290) 128 in one, which halves
-// the decodes of experts with many positions.
+// the decodes of experts with many positions. A constant of the type, a compromise over the token counts. Q4_K's launch, 64
+// and 128: 74 and 85 us at 37 tokens, 166 and 170 at 2048. Whole forwards, 2560 x 640 over 512 experts, 64 and 128:
+//   tokens             37 even    1000 even   1000 Zipf   4096 even    4096 Zipf
+//   IQ3_XXS            353 361    656 681     484 470     1490 1343    1310 1241
+//   IQ3_S              365 372    685 715     495 480     1558 1417    1359 1304
+//   IQ4_XS             364 370    692 704     491 472     1577 1398    1377 1282
+//   IQ2_S              311 319    583 606     438 435     1387 1281    1195 1178
 template <uint32_t kType>
 constexpr uint32_t plane_pos() { return kType == QT_Q4_K || kType == QT_IQ2_S ? 64u : 128u; }
 

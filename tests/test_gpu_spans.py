@@ -113,6 +113,31 @@ def test_spans_tiny_scales(gt):
     check(gt, NL, 1024, 256, h.CODEBOOKS, scales=np.exp2([0.0, 0.0, -20.0, -85.0, -95.0, -105.0, -118.0]))
 
 
+@pytest.mark.parametrize("gt,dt", [(Q4, NL), (I3, Q2), (XX, Q8), (S2, NL), (XS, Q8)], ids=lambda v: moe.TYPE_NAMES[v])
+def test_spans_infinite_scales(gt, dt):
+    """Blocks whose scale is infinite in rows of up (the SwiGLU limit makes their values finite again) and, infinite or NaN, in
+    rows of down: no other row or position sees them."""
+    say("spans, infinite scales", (moe.TYPE_NAMES[gt], moe.TYPE_NAMES[dt]))
+    H, F, T, E, limit = 512, 256, 70, 3, 0.05
+    L = h.Layer(H, F, E, E, gt, dt, has_shared=False, seed=970 + gt, swiglu_limit=limit)
+    x = h.tokens(971, T, H)
+    jobs = [(L.experts[e], t, 0.5 + e) for t in range(T) for e in range(E) if (t + e) % 5]
+    clean = h.orc_compute_many(gt, dt, H, F, jobs, x, swiglu_limit=limit)
+    up, down = (L.experts[1][m].reshape((F, H)[m - 1], -1) for m in (1, 2))
+    up[[5, 100], :2] = 0x00, 0x7C
+    yo = h.orc_compute_many(gt, dt, H, F, jobs, x, swiglu_limit=limit)
+    assert np.isfinite(yo).all() and not np.array_equal(yo, clean)
+    down[[7, 300], :2], down[33, :2] = (0x00, 0xFC), (0x00, 0x7E)
+    yo = h.orc_compute_many(gt, dt, H, F, jobs, x, swiglu_limit=limit)
+    assert np.isfinite(np.delete(yo, [7, 300, 33], axis=1)).all() and np.isinf(yo[:, 7]).any() and np.isnan(yo[:, 33]).any()
+    blk = moe.MoeBlock(H, F, 8, E, gt, dt, False, max_tokens=T, swiglu_limit=limit)
+    if gt in moe.CODEBOOK_TYPES:
+        blk.set_codebooks(h.CODEBOOKS)
+    y = blk.compute_many(jobs, x)
+    blk.close()
+    assert np.array_equal(y, yo, equal_nan=True)
+
+
 @pytest.mark.parametrize("gt", [XX, S2], ids=lambda v: moe.TYPE_NAMES[v])
 def test_codebooks_past_the_levels(gt):
     """A caller's tables whose bytes take more values than the planes' digit tables hold run the general path."""
