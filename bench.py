@@ -1,8 +1,8 @@
-"""Benchmark of the MoE block on one MI355X (BASELINE.json's metric on its configs).
+"""Benchmark of the MoE block on one MI355X.
 
 A step is one forward of the block (router, experts, shared expert, combine) over one batch of synthetic tokens,
-inputs resident in HBM. The default run measures both halves of BASELINE's metric and prints them in one JSON line:
-  - decode (the line's value): BASELINE.json configs[1] (config 2), the speculative-verify batch of 8 tokens, Q4_K
+inputs resident in HBM. The default run measures both halves of the metric and prints them in one JSON line:
+  - decode (the line's value): config 2, the speculative-verify batch of 8 tokens, Q4_K
     experts, hidden 2048, 512 experts, top-10 + shared, intermediate 512, Zipf(1.1) logit bias; roofline: HBM GB/s;
   - prefill (the "prefill" object): config 4, one 2048-token chunk, Q4_K, Zipf(1.1); roofline: the routed gate/up
     launch's int8 MFMA rate.
@@ -13,7 +13,7 @@ Cache defeat (decode): the MI355X's 256 MB Infinity Cache would hold one layer's
 resident as several layers (independent routers and biases, so each step routes differently) whose touched bytes,
 counted from each layer's own routing, sum past 512 MB; step i runs layer i mod n_layers.
 
---config picks one of BASELINE's configs alone: decode 1, 2, 3, 3b; prefill 4; the 48-layer stack 5 (decode) and
+--config picks one configuration alone: decode 1, 2, 3, 3b; prefill 4; the 48-layer stack 5 (decode) and
 5p (prefill, two chunks of 2048).
 """
 import argparse
@@ -38,7 +38,7 @@ CONFIGS = {
               types=(21, 12, 8, 8), T=1, zipf=1.1, layers=48),
     "5p": dict(name="config5: 48-layer stack, prefill 4096 tokens in 2 chunks of 2048, gate/up IQ3_S, down Q4_K, "
                     "shared Q8_0, Zipf(1.1) per layer", types=(21, 12, 8, 8), T=4096, chunk=2048, zipf=1.1, layers=48),
-    # Not a BASELINE config: config 4's block with the hyper-connection mix and combine around it (moe_forward_hc), a
+    # Beside the numbered configurations: config 4's block with the hyper-connection mix and combine around it (moe_forward_hc), a
     # low rank of 256 at this n_embd (the model's 320 at 2560 scaled); its own JSON line, never the headline.
     "hc": dict(name="config4 + hyper-connection mix and combine (hc_lr 256): prefill T=2048, Q4_K, Zipf(1.1)",
                types=(12, 12, 12, 12), T=2048, zipf=1.1, hc_lr=256),

@@ -1,5 +1,5 @@
 /* TEST INFRASTRUCTURE - the CPU oracle of the MoE block. Not product code: only tests/, __graft_entry__.smoke() and
- * bench.py's cpu_baseline leg load it, as the checker; the product (c0ven_amd/) never links or calls it.
+ * bench.py's cpu_baseline leg load it; the product (c0ven_amd/) never links or calls it.
  *
  * A plain-C restatement of the reference's CPU expert path and of the block around it:
  *   - the weight decoders (ggml's dequantize_row_q8_0 / _q4_K / _q5_K / _q6_K / _iq3_s / _iq4_nl / _iq4_xs / _q2_0 /

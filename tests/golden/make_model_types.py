@@ -1,7 +1,7 @@
 """Writes tests/golden/model_layer_types.json: the MoE tensors' types and shapes of every block of the reference's
 model file, read from the reference's census docs/model/tensors-IQ3_S.tsv (a data file: name, type, ggml type,
-shape, bytes, shard, offset, category). Run in a checkout that has the reference at /root/reference; the GPU box and
-the tests read only the JSON it writes."""
+shape, bytes, shard, offset, category). Run in a checkout that has the reference at /root/reference; the
+tests read only the JSON it writes."""
 import collections
 import json
 import os

@@ -1,4 +1,4 @@
-"""Shared test helpers: the CPU oracle's bindings (oracle/liboracle.so, the checker), synthetic layers drawn with the
+"""Shared test helpers: the CPU oracle's bindings (oracle/liboracle.so), synthetic layers drawn with the
 library's seeded generator, and the parity metrics.
 
 The oracle is test infrastructure: it is loaded here, by the tests, smoke() and bench.py's cpu_baseline, and by
@@ -325,7 +325,7 @@ def max_abs(a, b):
     return float(np.max(np.abs(np.asarray(a, np.float64) - np.asarray(b, np.float64))))
 
 
-# The block's bar (north_star): top-k ids bit-exact, y within max-abs 1e-3 and rel-L2 1e-4. The prefill path's
+# The block's bar: top-k ids bit-exact, y within max-abs 1e-3 and rel-L2 1e-4. The prefill path's
 # default router gives the oracle's ids with logits within ~1e-6 of its own, so its weights are held to W_TOL.
 TOL_ABS, TOL_REL, W_TOL = 1e-3, 1e-4, 2e-5
 

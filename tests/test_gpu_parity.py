@@ -1,6 +1,6 @@
 """The HIP path against the CPU oracle, through the C ABI (libc0ven_moe.so), on the GPU.
 
-The bar (north_star): top-k expert ids and decoded weight blocks bit-exact; the block's output within max-abs 1e-3
+The bar: top-k expert ids and decoded weight blocks bit-exact; the block's output within max-abs 1e-3
 and rel-L2 1e-4. The decode path reproduces the oracle's every rounding (its ORACLE ORDER, libm's expf), so these
 tests also hold its output to bit equality, and report the distance when it is not.
 """

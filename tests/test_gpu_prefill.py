@@ -5,7 +5,7 @@ With the exact router (MOE_FLAG_EXACT_ROUTER) it reproduces the oracle's every r
 held to bit equality; with the default matrix-core router the ids are still the oracle's (its top k are certified, and
 summed exactly where the bound leaves them open) and w, y are held to the bar (max-abs 1e-3, rel-L2 1e-4; w 2e-5). The dispatch is checked against a stable counting sort in numpy: the
 MoeTiles (shared/moe_tile.h:11-18) cover each expert's assignments in token order, at most MOE_TILE rows a tile.
-At BASELINE's config 4 size (2048 tokens, 512 experts, top-10) the oracle runs on a sample of the tokens, since each
+At config 4's size (2048 tokens, 512 experts, top-10) the oracle runs on a sample of the tokens, since each
 token's output depends on that token alone.
 """
 import sys
@@ -141,7 +141,7 @@ def test_prefill_forwards_in_a_row():
 
 @pytest.mark.parametrize("exact", ROUTERS)
 def test_prefill_config4_sampled(exact):
-    """2048 tokens, H 2048, F 512, 512 experts, top-10 + shared, Q4_K, Zipf(1.1)."""
+    """Config 4: 2048 tokens, H 2048, F 512, 512 experts, top-10 + shared, Q4_K, Zipf(1.1)."""
     say("prefill config 4, exact router", exact)
     L = h.Layer(2048, 512, 512, 10, Q4, Q4, seed=2026, zipf=1.1, nthreads=0)
     blk = L.block(max_tokens=2048, exact_router=exact)
@@ -188,7 +188,7 @@ def test_prefill_dispatch_many_windows():
 
 
 def test_prefill_config5_chunk_sampled():
-    """BASELINE config 5's layer at full size, one 2048-token prefill chunk: H 2048, F 512, 512 experts, top-10,
+    """Config 5's layer at full size, one 2048-token prefill chunk: H 2048, F 512, 512 experts, top-10,
     gate/up IQ3_S, down Q4_K, shared expert Q8_0, Zipf(1.1). Hot experts span many 64-row tiles. ids and w on every
     token, y on a sample (each token's y depends on that token alone)."""
     say("prefill config 5 chunk")

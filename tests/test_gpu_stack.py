@@ -1,4 +1,4 @@
-"""A stack of MoE blocks (BASELINE config 5's shape: gate/up IQ3_S, down Q4_K, shared expert Q8_0, H 2048, F 512,
+"""A stack of MoE blocks (config 5's shape: gate/up IQ3_S, down Q4_K, shared expert Q8_0, H 2048, F 512,
 512 experts, top-10, each layer with its own router and Zipf(1.1) bias) against the CPU oracle, through the C ABI.
 
 Attention and DeltaNet are omitted, as in config 5; a residual x <- x + y (numpy, fp32, the same on both sides) links

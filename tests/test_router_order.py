@@ -1,4 +1,4 @@
-"""Two summation orders the router's parity rests on, measured on the CPU at BASELINE config 2's router (H 2048,
+"""Two summation orders the router's parity rests on, measured on the CPU at config 2's router (H 2048,
 512 experts + the shared gate, top-10, N(0, 0.02) bf16 weights, N(0, 1) tokens, Zipf(1.1) logit bias).
 
 1. Router logits. The oracle (and both GPU paths) round the exact fp64 sum of the bf16 products once to fp32. ggml's
