@@ -281,7 +281,8 @@ MOE_API moe_status moe_dequantize(moe_ctx *ctx, uint32_t type, const uint8_t *bl
  * iq3xxs_grid are taken from it (this build does not carry them); its IQ3_S region must equal ggml's iq3s_grid, the
  * check that the buffer has the layout. A context whose types include IQ3_XXS or IQ2_S refuses forwards and
  * moe_dequantize of those types until this is called. No counterpart call in the reference, whose kernels receive the
- * same buffer at load time. */
+ * same buffer at load time. Set them before forwards are captured into a graph: the kernels of a prefill call are chosen by
+ * the tables (at most four byte values in iq2s_grid and eight in iq3xxs_grid, as ggml's have, or more). */
 MOE_API moe_status moe_set_codebooks(moe_ctx *ctx, const uint8_t *qgrid, uint64_t bytes);
 
 /* Synthetic inputs (seeded, so that every machine draws the same values): counter-based normals, the library's
